@@ -382,10 +382,11 @@ int ph_server_result(ph_server* s, int job, float* rgb) {
         PH_CHECK(hipStreamSynchronize(s->stream()));
         const float inv = 1.0f / float(j.desc.spp);
         for (size_t i = 0; i < n; i++) {
-            // The partial images in sub-stream order (one plane: the accumulation itself).
-            float r = raw[i].x, g = raw[i].y, b = raw[i].z;
+            // The pixel's partial sums in sub-stream order (one: the accumulation itself).
+            const float4* part = raw.data() + i * size_t(j.split);
+            float r = part->x, g = part->y, b = part->z;
             for (int p = 1; p < j.split; p++) {
-                const float4& v = raw[size_t(p) * n + i];
+                const float4& v = part[p];
                 r += v.x;
                 g += v.y;
                 b += v.z;

@@ -228,6 +228,21 @@ PH_DEV uint8_t term_stage(const JobParams& jp, const State& st, int slot) {
     return uint8_t(S_TERM | (st.sample[slot] + 1 >= end ? S_NEED : 0));
 }
 
+// Where the slot's sub-stream sums its samples: the partial sums of a pixel follow each other (a wave's
+// slots run neighbouring sub-streams of the same pixels, so that their sums share cache lines).
+template <bool Multi>
+PH_DEV int accum_index(const JobParams& jp, const State& st, int slot, int pixel) {
+    return (Multi || jp.split > 1) ? pixel * jp.split + st.part[slot] : pixel;
+}
+
+// The sum so far. A single render's sub-stream starts from nothing at its first sample: its partial sum
+// is not read there (nor cleared beforehand).
+template <bool Multi>
+PH_DEV float4 partial_sum(const JobParams& jp, const State& st, int slot, int k, const float4* acc) {
+    if (!Multi && jp.split > 1 && k == st.part[slot] * jp.span) return make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    return *acc;
+}
+
 PH_DEV void start_sample(const JobParams& jp, const State& st, int slot, int pixel, int k) {
     const int x = pixel % jp.width, y = pixel / jp.width;
     Pcg rng = pixel_rng(uint32_t(pixel), jp.frame0 + uint32_t(k), jp.seed);
@@ -253,18 +268,22 @@ PH_DEV void start_work(const Work& work, const State& st, int chunks, int slot, 
     int local = int(w - (Multi ? work.chunk_first[c] : 0)) + pass.w;
     int k0 = pass.y;
     if (Multi) {
-        // Items of a pass: sub-stream `part` of every pixel, for parts 0 .. split-1 in turn; the pass's
-        // sample range is relative to the sub-stream's first sample.
-        const int part = local / jp.pixels;
-        local -= part * jp.pixels;
+        // Items of a pass: the sub-streams of each pixel, pixel after pixel; the pass's sample range is
+        // relative to the sub-stream's first sample.
+        const int part = int(uint32_t(local) % uint32_t(jp.split));
+        local = int(uint32_t(local) / uint32_t(jp.split));
         k0 += part * jp.span;
         st.job[slot] = pass.x;
         st.part[slot] = part;
         st.sample_end[slot] = part * jp.span + pass.z;
     } else if (jp.split > 1) {
-        // A single render in sub-streams: item = part * pixels + pixel item; the part's samples in order.
-        const int part = local / jp.pixels;
-        local -= part * jp.pixels;
+        // A single render in sub-streams: item = pixel item * split + part; the part's samples in order. The
+        // sub-streams of a pixel are neighbours, so a wave of 64 one-sample sub-streams traces 64 camera rays
+        // of one pixel, and the paths in flight cover a quarter of the image's tiles, not all of them: traversal
+        // lanes walk the same nodes, and more of them stay in the L2. 1080p, 64 samples, 1M triangles: 94.2 ms
+        // against 101.9 with sub-stream 0 of every pixel first (with the partial sums laid out to match).
+        const int part = int(uint32_t(local) % uint32_t(jp.split));
+        local = int(uint32_t(local) / uint32_t(jp.split));
         k0 = part * jp.span;
         st.part[slot] = part;
         st.sample_end[slot] = k0 + jp.span;
@@ -741,8 +760,8 @@ __global__ __launch_bounds__(256) void regen_kernel(Work work, State st, int* co
             f3 L = xyz(ld_stream(st.L + slot));
             if (!finite3(L) || L.x < 0 || L.y < 0 || L.z < 0) L = mk3(0);
             const bool parts = Multi || jp.split > 1;
-            float4* acc = jp.accum + (parts ? st.part[slot] * jp.pixels : 0) + pixel;
-            float4 a = *acc;
+            float4* acc = jp.accum + accum_index<Multi>(jp, st, slot, pixel);
+            float4 a = partial_sum<Multi>(jp, st, slot, k, acc);
             a.x += L.x;
             a.y += L.y;
             a.z += L.z;
@@ -819,8 +838,8 @@ __global__ __launch_bounds__(kFinishBlock) __attribute__((amdgpu_waves_per_eu(4)
                 pixel = st.pixel[slot];
                 k = st.sample[slot];
                 end = parts ? st.sample_end[slot] : jp.spp;
-                acc = jp.accum + (parts ? st.part[slot] * jp.pixels : 0) + pixel;
-                a = *acc;
+                acc = jp.accum + accum_index<false>(jp, st, slot, pixel);
+                a = partial_sum<false>(jp, st, slot, k, acc);
                 live = true;
                 resumed = false;
             }
@@ -873,19 +892,33 @@ __global__ void finish_clear_kernel(int* counters, const unsigned long long* ite
 }
 
 // The end of a single render in sub-streams: adds the partial sums to the accumulation, sub-stream 0
-// first.
-__global__ void add_parts_kernel(const float4* parts, int pixels, int count, float4* accum) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= pixels) return;
-    float4 a = accum[i];
-    for (int p = 0; p < count; p++) {
-        const float4 s = parts[size_t(p) * size_t(pixels) + size_t(i)];
-        a.x += s.x;
-        a.y += s.y;
-        a.z += s.z;
-        a.w += s.w;
+// first. The sums of a pixel are consecutive: a block stages those of kPartPixels pixels in LDS, kPartRun
+// of each at a time, with coalesced loads, and one lane per pixel and component adds them in order. The
+// rows are padded by one entry, so that the lanes of a step read different banks.
+constexpr int kPartPixels = 16, kPartRun = 64, kPartThreads = 256;
+
+__global__ __launch_bounds__(kPartThreads) void add_parts_kernel(const float4* parts, int pixels, int count, float4* accum) {
+    __shared__ float4 tile[kPartPixels * (kPartRun + 1)];
+    const int first = blockIdx.x * kPartPixels;
+    const int n = min(kPartPixels, pixels - first);
+    const int t = threadIdx.x;
+    const bool sums = t < 4 * n;
+    float* out = reinterpret_cast<float*>(accum + first);
+    float a = sums ? out[t] : 0.0f;
+    for (int p0 = 0; p0 < count; p0 += kPartRun) {
+        const int run = min(kPartRun, count - p0);
+        for (int e = t; e < n * run; e += kPartThreads) {
+            const int i = e / run, p = e - i * run;
+            tile[i * (kPartRun + 1) + p] = ld_stream(parts + size_t(first + i) * size_t(count) + size_t(p0 + p));
+        }
+        __syncthreads();
+        if (sums) {
+            const float* row = reinterpret_cast<const float*>(tile + (t >> 2) * (kPartRun + 1)) + (t & 3);
+            for (int p = 0; p < run; p++) a += row[4 * p];
+        }
+        __syncthreads();
     }
-    accum[i] = a;
+    if (sums) out[t] = a;
 }
 
 int device_cus() {
@@ -1286,7 +1319,6 @@ void WavefrontEngine::render(hipStream_t st, const WavefrontJob& job, bool count
     sub.split = split;
     if (split > 1) {
         m.part_sums.allocate(size_t(items));
-        m.part_sums.zero(st);
         sub.accum = m.part_sums.ptr;
     }
     const JobParams jp = m.params_of(sub, job.mat_class ? job.mat_class : m.mat_class.ptr);
@@ -1316,7 +1348,8 @@ void WavefrontEngine::render(hipStream_t st, const WavefrontJob& job, bool count
         if (iterations > bound) throw std::runtime_error("wavefront loop did not drain");
     }
     if (split > 1) {
-        hipLaunchKernelGGL(add_parts_kernel, dim3((pixels + 255) / 256), dim3(256), 0, st, m.part_sums.ptr, pixels, split, job.accum);
+        hipLaunchKernelGGL(add_parts_kernel, dim3((pixels + kPartPixels - 1) / kPartPixels), dim3(kPartThreads), 0, st, m.part_sums.ptr, pixels,
+                           split, job.accum);
         PH_CHECK(hipGetLastError());
     }
     TraceTotals tot[2] = {};
