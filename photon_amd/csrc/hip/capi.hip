@@ -572,7 +572,11 @@ int ph_trace(ph_renderer* r, const ph_ray* rays, int n, int anyhit, ph_hit* hits
     if (!r->uploaded) return fail("no scene uploaded");
     return guarded([&] {
         ph_renderer& m = *r;
-        if (!launch_trace(m.stream, m.view, rays, n, anyhit != 0, hits, counts, 128, 32, false, 0, 0))
+        // Closest hits do not depend on the walk, so they go over the wide nodes. Any-hit results are the first hit of
+        // the binary walk's order, and counts are its counts.
+        if (m.view.wide && !anyhit && !counts)
+            launch_trace_wide(m.stream, m.view, rays, n, hits);
+        else if (!launch_trace(m.stream, m.view, rays, n, anyhit != 0, hits, counts, 128, 32, false, 0, 0))
             return fail("unsupported traversal launch shape");
         PH_CHECK(hipStreamSynchronize(m.stream));
         return 0;

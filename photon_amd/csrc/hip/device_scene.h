@@ -56,7 +56,7 @@ public:
     bool ready() const { return ready_; }
     size_t bytes() const {
         size_t b = 0;
-        b += nodes_.bytes() + tris_.bytes() + materials_.bytes() + indices_.bytes() + tri_emissive_.bytes();
+        b += nodes_.bytes() + wide_.bytes() + tris_.bytes() + materials_.bytes() + indices_.bytes() + tri_emissive_.bytes();
         b += normals_.bytes() + uvs_.bytes() + tangents_.bytes() + srgb_lut_.bytes() + env_texels_.bytes();
         b += env_marginal_.bytes() + env_conditional_.bytes() + textures_.bytes() + texels_.bytes();
         b += guide_marginal_.bytes() + guide_conditional_.bytes();
@@ -91,9 +91,12 @@ public:
         texels_.upload(d.texels, size_t(d.num_texels), st);
         srgb_lut_.upload(d.srgb_lut, 256, st);
         punctual_.upload(d.punctual, size_t(d.num_punctual), st);
-        upload_lights(d, st);
         phd::DScene& v = view_;
         v.nodes = or_null(nodes_);
+        v.num_nodes = d.num_nodes;
+        upload_lights(d, st);
+        build_wide_nodes(st, nodes_.ptr, d.num_nodes, d.num_tris, wide_);
+        v.wide = or_null(wide_);
         v.indices = or_null(indices_);
         v.normals = or_null(normals_);
         v.uvs = or_null(uvs_);
@@ -103,7 +106,6 @@ public:
         v.srgb_lut = or_null(srgb_lut_);
         v.punctual = or_null(punctual_);
         v.num_tris = d.num_tris;
-        v.num_nodes = d.num_nodes;
         v.top_nodes = top;
         v.num_punctual = d.num_punctual;
         v.num_textures = d.num_textures;
@@ -116,6 +118,7 @@ public:
     // Re-uploads what a light rebuild changes (GpuRenderer::update_lights, gpu_renderer.cu:299-334).
     void upload_lights(const ph_scene_desc& d, hipStream_t st) {
         tris_.upload(d.tris, size_t(d.num_tris) * 3, st);
+        if (d.num_tris > 0) mark_leaves(st, nodes_.ptr, view_.num_nodes, d.num_tris, tris_.ptr);
         materials_.upload(d.materials, size_t(d.num_materials) * 5, st);
         emissive_.upload(d.emissive, size_t(d.num_emissive), st);
         tri_emissive_.upload(d.tri_emissive, d.tri_emissive ? size_t(d.num_tris) : 0, st);
@@ -167,7 +170,7 @@ public:
     }
 
 private:
-    DevBuf<float4> nodes_, tris_, materials_;
+    DevBuf<float4> nodes_, wide_, tris_, materials_;
     DevBuf<int> indices_, tri_emissive_;
     DevBuf<float> normals_, uvs_, tangents_, srgb_lut_, env_texels_, env_marginal_, env_conditional_;
     DevBuf<int> guide_marginal_, guide_conditional_;

@@ -4,7 +4,7 @@
 #pragma once
 
 #include "dshade.h"
-#include "dtrace.h"
+#include "dwide.h"
 
 namespace phd {
 
@@ -41,6 +41,22 @@ struct RayTally {
 // The path from its next extension ray (ro, rd) on, with the generator in the state it has at that
 // point: the remaining vertices exactly as a path that started here would run them. trace_path is the
 // whole path; the wavefront engine resumes its last paths in flight with this.
+// The stack of a kernel that traces whole paths: 16 KB of LDS per 128 lanes for either walk.
+template <int Block, bool Wide>
+using PathStack = StackShape<Block, Wide ? 20 : 32, Wide>;
+
+// A path's closest-hit and any-hit queries, over the wide nodes or (a scene outside their limits, or a
+// counting kernel) the binary ones: the answers are the same.
+template <bool AnyHit, bool Count, int Depth, int Block>
+PH_DEV bool path_query(const DScene& s, f3 o, f3 d, float tmax, HitRec& hit, WideStack<Depth, Block>& stack, TraceCount*) {
+    return traverse_wide<AnyHit, !AnyHit>(trace_scene(s), o, d, tmax, hit, stack);
+}
+
+template <bool AnyHit, bool Count, int Depth>
+PH_DEV bool path_query(const DScene& s, f3 o, f3 d, float tmax, HitRec& hit, LaneStack<Depth>& stack, TraceCount* cnt) {
+    return traverse<AnyHit, Count>(s, o, d, tmax, hit, stack, cnt);
+}
+
 template <class Stack, bool Count>
 PH_DEV f3 trace_path_from(const DScene& s, f3 ro, f3 rd, Pcg& rng, const PathOpts& opt, PathState ps, PrimaryOut* primary, Stack& stack,
                           TraceCount* cnt, RayTally* tally) {
@@ -51,7 +67,7 @@ PH_DEV f3 trace_path_from(const DScene& s, f3 ro, f3 rd, Pcg& rng, const PathOpt
     for (int depth = ps.depth;; depth++) {
         HitRec hit{kInf, -1, 0.0f, 0.0f};
         if (tally) tally->ext++;
-        if (!traverse<false, Count>(s, ro, rd, kInf, hit, stack, cnt)) {
+        if (!path_query<false, Count>(s, ro, rd, kInf, hit, stack, cnt)) {
             f3 le = sky_radiance(s, rd);
             float w = (prev_delta || s.p_env <= 0) ? 1.0f : mis_power(prev_pdf, sky_pdf(s, rd));
             L = L + clamp_contribution(beta * le * w, depth, opt.clamp);
@@ -99,7 +115,7 @@ PH_DEV f3 trace_path_from(const DScene& s, f3 ro, f3 rd, Pcg& rng, const PathOpt
                     float stmax = ls.dist == kInf ? kInf : ls.dist * (1.0f - 1e-4f);
                     HitRec sh{kInf, -1, 0.0f, 0.0f};
                     if (tally) tally->shadow++;
-                    if (!traverse<true, Count>(s, so, ls.wi, stmax, sh, stack, cnt)) {
+                    if (!path_query<true, Count>(s, so, ls.wi, stmax, sh, stack, cnt)) {
                         float w = ls.delta ? 1.0f : mis_power(ls.pdf, pdf_b);
                         L = L + clamp_contribution(beta * f * fabsf(wi.z) * ls.radiance * (w / ls.pdf), depth, opt.clamp);
                     }

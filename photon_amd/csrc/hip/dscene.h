@@ -2,12 +2,14 @@
 //
 // Layout in HBM (one allocation per array, 256-byte aligned by the allocator):
 //   nodes      64 B each, read as four 16-byte loads (dual-box node: both children's bounds at once)
-//   tris       48 B each, BVH order (v0|material, e1|flags, e2|pad), three 16-byte loads
+//   wide       64 B each, the tree over four-wide quantised nodes (dwide.h)
+//   tris       48 B each, BVH order (v0|material, e1|flags, e2|leaf), three 16-byte loads; `leaf` (the padding word
+//              on the host) is the triangle's leaf as 2 * node + side
 //   indices    12 B per triangle; normals 12 B, uvs 8 B, tangents 16 B per vertex
 //   materials  80 B each, read as five 16-byte loads
 //   texels     RGBA8 pool; srgb_lut 256 floats
 //   emissive / tri_emissive / alias: light tables; env texels (12 B) and CDFs
-// The scene on the CPU side is identical byte for byte (include/photon_types.h).
+// The scene on the CPU side is otherwise identical byte for byte (include/photon_types.h).
 #pragma once
 
 #include "dmath.h"
@@ -17,6 +19,7 @@ namespace phd {
 
 struct DScene {
     const float4* nodes;
+    const float4* wide;  // the same tree over four-wide nodes (dwide.h); null where their limits are exceeded
     const float4* tris;
     const int* indices;
     const float* normals;

@@ -103,16 +103,18 @@ PH_DEV bool alpha_cut(const DScene& s, int tri, int material, float u, float v) 
 }
 
 // What traversal reads of a scene, held in registers: the node and triangle arrays, the whole scene
-// for the (rare) alpha tests, and optionally the top `top_n` nodes staged in LDS by the block.
+// for the (rare) alpha tests, optionally the top `top_n` nodes staged in LDS by the block, and the wide
+// nodes (dwide.h).
 struct TraceScene {
     const float4* nodes;
     const float4* tris;
     const DScene* full;
     const float4* top;
     int top_n;
+    const float4* wide;
 };
 
-PH_DEV TraceScene trace_scene(const DScene& s) { return TraceScene{s.nodes, s.tris, &s, nullptr, 0}; }
+PH_DEV TraceScene trace_scene(const DScene& s) { return TraceScene{s.nodes, s.tris, &s, nullptr, 0, s.wide}; }
 
 // Copies nodes [0, n) into the block's LDS array `top` (4 float4 per node). All threads call.
 PH_DEV void stage_top_nodes(float4* top, const float4* nodes, int n) {
@@ -262,44 +264,88 @@ PH_DEV WaveShare wave_share(int n, int xcd_parts) {
     return WaveShare{first, last - first, int(blockIdx.x / parts) * wpb + int(threadIdx.x >> 6), blocks_here * wpb};
 }
 
+// A walk over the binary nodes, in the form that trace_stream drives (WideWalk is the other one).
+template <bool AnyHit, bool Count>
+struct BinaryWalk {
+    static constexpr bool kSecond = false;  // every walk settles its answer
+    Walker w;
+    HitRec hit;
+    TraceCount cnt;
+    PH_DEV void start(f3 o, f3 d, float tmax) {
+        w = walker(o, d, tmax);
+        hit = HitRec{kInf, -1, 0.0f, 0.0f};
+    }
+    template <class Stack>
+    PH_DEV bool step(const TraceScene& ts, Stack& stack) {
+        return walk_step<AnyHit, Count>(ts, w, hit, stack, &cnt);
+    }
+    PH_DEV bool settled(const TraceScene&) const { return true; }
+    PH_DEV int material_of(const TraceScene& ts) const { return __float_as_int(ldg(ts.tris + 3 * hit.tri).w); }
+};
+
 // Persistent traversal of entries [0, n) with lane refill. A lane whose ray is finished takes the next
 // entry of its wave's share as soon as at least `refill` lanes of the wave are free (or all are), so a
 // wave is not held by its slowest ray; the wave leaves when its share is drained and none of its lanes
 // has a ray. Each ray is walked exactly as traverse() walks it: only the lane it runs on and the moment
-// it starts change. `load(i, ts, w, hit)` starts entry i (and may set the lane's scene);
-// `finish(ts, w, hit)` stores its result.
-template <bool AnyHit, bool Count, class Stack, class Load, class Finish>
-PH_DEV void trace_stream(int n, int parts, int refill, TraceScene ts, Stack& stack, TraceCount& cnt, Load load, Finish finish) {
+// it starts change. `ray_of(i)` is entry i's ray (>= 0), `load(ray, ts, walk)` starts it (and may set the
+// lane's scene) and `finish(ray, ts, walk)` stores its result.
+// Results are stored when lanes are refilled, not as each ray ends: rays end in nearly every step, and each
+// time the whole wave would issue the storing code and wait for its dependent loads.
+// A ray whose walk has not settled its answer keeps its lane free until the wave has no ray left; then such
+// rays are traced over the binary nodes together. Inside the loop that second walk's registers would come on
+// top of the first's (84 instead of 64, 5 waves per SIMD instead of 8).
+template <bool AnyHit, class Walk, class Stack, class RayOf, class Load, class Finish>
+PH_DEV void trace_stream(int n, int parts, int refill, TraceScene ts, Stack& stack, Walk& walk, RayOf ray_of, Load load, Finish finish) {
     const WaveShare ws = wave_share(n, parts);
     int pos = 0;  // entries of this wave's share already handed to lanes
     bool drained = ws.wave >= ws.batches;
-    bool live = false;
-    Walker w{};
-    HitRec hit{};
-    for (;;) {
-        if (!drained) {
-            const uint64_t need = __ballot(!live);
-            const int k = __popcll(need);
-            if (k >= refill || k == 64) {
-                if (!live) {
-                    const int j = pos + __popcll(need & ((1ull << __lane_id()) - 1ull));
-                    const int b = ws.wave + (j >> 6) * ws.waves;
-                    const int i = (ws.first + b) * 64 + (j & 63);
-                    if (b < ws.batches && i < n) {
-                        load(i, ts, w, hit);
-                        live = true;
+    do {
+        bool live = false;
+        int ray = -1;  // this lane's; -2 - ray once it is to be traced again
+        for (;;) {
+            const uint64_t free = __ballot(!live && ray >= -1);
+            const bool none = __ballot(live) == 0;
+            if (none || (!drained && __popcll(free) >= refill)) {
+                if (!live && ray >= 0) {
+                    if (walk.settled(ts)) {
+                        finish(ray, ts, walk);
+                        ray = -1;
+                    } else {
+                        ray = -2 - ray;
                     }
                 }
-                pos += k;
-                if (ws.wave + (pos >> 6) * ws.waves >= ws.batches) drained = true;
+                if (!drained) {
+                    const uint64_t need = __ballot(!live && ray == -1);
+                    if (!live && ray == -1) {
+                        const int j = pos + __popcll(need & ((1ull << __lane_id()) - 1ull));
+                        const int b = ws.wave + (j >> 6) * ws.waves;
+                        const int i = (ws.first + b) * 64 + (j & 63);
+                        if (b < ws.batches && i < n) {
+                            ray = ray_of(i);
+                            load(ray, ts, walk);
+                            live = true;
+                        }
+                    }
+                    pos += __popcll(need);
+                    if (ws.wave + (pos >> 6) * ws.waves >= ws.batches) drained = true;
+                }
+                if (__ballot(live) == 0) break;
             }
+            if (live && !walk.step(ts, stack)) live = false;
         }
-        if (__ballot(live) == 0) break;
-        if (live && !walk_step<AnyHit, Count>(ts, w, hit, stack, &cnt)) {
-            finish(ts, w, hit);
-            live = false;
+        if constexpr (Walk::kSecond) {
+            if (ray < -1) {
+                ray = -2 - ray;
+                auto s = stack.binary();
+                BinaryWalk<AnyHit, false> again;
+                load(ray, ts, again);
+                while (again.step(ts, s)) {
+                }
+                finish(ray, ts, again);
+            }
+            walk = Walk{};
         }
-    }
+    } while (!drained);
 }
 
 template <bool AnyHit, bool Count, class Stack>

@@ -95,6 +95,13 @@ void launch_sample(hipStream_t st, const phd::DScene& s, const ph_camera_view& c
 int64_t bvh_build_device(const float* positions, int num_vertices, const int* indices, int n, int bins, int max_leaf, float traversal_cost,
                          ph_bvh_node* nodes_out, int* order_out, ph_bvh_build_stats& stats);
 
+// ---- wide_build.hip -----------------------------------------------------------------------------------
+// The scene's four-wide nodes (dwide.h) from its binary nodes. False, with `wide` empty, where the format's limits
+// (leaf size, triangle count, coordinates) are exceeded: such a scene is traced over the binary nodes.
+bool build_wide_nodes(hipStream_t st, const float4* nodes, int num_nodes, int num_tris, DevBuf<float4>& wide);
+// Writes each triangle's leaf into the triangle's unused word.
+void mark_leaves(hipStream_t st, const float4* nodes, int num_nodes, int num_tris, float4* tris);
+
 // Guide tables of `rows` CDFs of n + 1 entries each (row r at cdf + r * stride): guide[r * (m + 1) + k]
 // is the index the CDF search returns for u = k / m (m a power of two).
 void build_cdf_guides(hipStream_t st, const float* cdf, int rows, int n, size_t stride, int m, int* guide);
@@ -109,5 +116,8 @@ void launch_display(hipStream_t st, const DisplayParams& p, const float4* accum,
 // Persistent launches stage the top `lds_nodes` BVH nodes in each block's LDS.
 bool launch_trace(hipStream_t st, const phd::DScene& s, const ph_ray* rays, int n, bool anyhit, ph_hit* hits, uint32_t* counts, int block, int depth,
                   bool persistent, int lds_nodes, int grid_blocks);
+
+// Closest hits over the wide nodes, which the scene must have.
+void launch_trace_wide(hipStream_t st, const phd::DScene& s, const ph_ray* rays, int n, ph_hit* hits);
 
 }  // namespace phk

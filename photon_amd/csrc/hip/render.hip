@@ -11,7 +11,7 @@ namespace phk {
 namespace {
 
 constexpr int kBX = 16, kBY = 8, kPixelBlock = kBX * kBY;
-constexpr int kMegaDepth = 32;  // LDS stack entries per lane in the per-pixel kernels
+constexpr int kMegaDepth = 32;  // LDS stack entries per lane of the heat map
 // Waves per SIMD the per-pixel kernels are compiled for. The whole integrator is live in one kernel,
 // and left alone the compiler gives it registers for 2 waves per SIMD (228-246 VGPRs), too few to hide
 // the traversal's memory latency. At 4 (128 VGPRs, the rest spilled), with bit-identical output:
@@ -20,19 +20,21 @@ constexpr int kMegaDepth = 32;  // LDS stack entries per lane in the per-pixel k
 //   * the 1080p render of that field runs at 479 Msamples/s instead of 329 (3 waves: 416).
 constexpr int kSampleWaves = 4;
 
+template <bool Wide>
 __global__ __launch_bounds__(kPixelBlock) __attribute__((amdgpu_waves_per_eu(kSampleWaves))) void render_kernel(DScene s, ph_camera_view cam, int w, int h, uint32_t frame0, int spp, uint32_t seed,
                                                              PathOpts opt, float4* accum, float4* albedo, float4* nd) {
-    __shared__ int lds[kMegaDepth * kPixelBlock];
+    using Shape = PathStack<kPixelBlock, Wide>;
+    __shared__ int lds[Shape::kWords];
     const int tid = threadIdx.y * kBX + threadIdx.x;
-    SpillArea<kMegaDepth> spill;
-    LaneStack<kMegaDepth> stack{lds + tid, kPixelBlock, spill.v};
+    typename Shape::Spill spill;
+    auto stack = Shape::make(lds, tid, spill);
     const int x = blockIdx.x * kBX + threadIdx.x, y = blockIdx.y * kBY + threadIdx.y;
     if (x >= w || y >= h) return;
     const int i = y * w + x;
     float4 a = accum[i];
     for (int k = 0; k < spp; k++) {
         PrimaryOut prim{mk3(0), 0.0f, mk3(0), -1, mk3(1), mk3(0)};
-        f3 L = pixel_sample<LaneStack<kMegaDepth>, false>(s, cam, x, y, w, h, frame0 + uint32_t(k), seed, opt, k == 0 ? &prim : nullptr, stack,
+        f3 L = pixel_sample<typename Shape::Stack, false>(s, cam, x, y, w, h, frame0 + uint32_t(k), seed, opt, k == 0 ? &prim : nullptr, stack,
                                                           nullptr);
         a.x += L.x;
         a.y += L.y;
@@ -47,17 +49,19 @@ __global__ __launch_bounds__(kPixelBlock) __attribute__((amdgpu_waves_per_eu(kSa
     accum[i] = a;
 }
 
+template <bool Wide>
 __global__ __launch_bounds__(kPixelBlock) __attribute__((amdgpu_waves_per_eu(kSampleWaves))) void sample_kernel(DScene s, ph_camera_view cam, int w, int h, uint32_t frame, uint32_t seed, PathOpts opt,
                                                              float4* color, float4* albedo, float4* nd, float4* position, float4* emission) {
-    __shared__ int lds[kMegaDepth * kPixelBlock];
+    using Shape = PathStack<kPixelBlock, Wide>;
+    __shared__ int lds[Shape::kWords];
     const int tid = threadIdx.y * kBX + threadIdx.x;
-    SpillArea<kMegaDepth> spill;
-    LaneStack<kMegaDepth> stack{lds + tid, kPixelBlock, spill.v};
+    typename Shape::Spill spill;
+    auto stack = Shape::make(lds, tid, spill);
     const int x = blockIdx.x * kBX + threadIdx.x, y = blockIdx.y * kBY + threadIdx.y;
     if (x >= w || y >= h) return;
     const int i = y * w + x;
     PrimaryOut p{mk3(0), 0.0f, mk3(0), -1, mk3(1), mk3(0)};
-    f3 L = pixel_sample<LaneStack<kMegaDepth>, false>(s, cam, x, y, w, h, frame, seed, opt, &p, stack, nullptr);
+    f3 L = pixel_sample<typename Shape::Stack, false>(s, cam, x, y, w, h, frame, seed, opt, &p, stack, nullptr);
     color[i] = make_float4(L.x, L.y, L.z, 1.0f);
     albedo[i] = make_float4(p.albedo.x, p.albedo.y, p.albedo.z, 1.0f);
     nd[i] = make_float4(p.normal.x, p.normal.y, p.normal.z, p.depth);
@@ -66,18 +70,20 @@ __global__ __launch_bounds__(kPixelBlock) __attribute__((amdgpu_waves_per_eu(kSa
 }
 
 // sample_kernel's sample, written as the compact G-buffer.
+template <bool Wide>
 __global__ __launch_bounds__(kPixelBlock) __attribute__((amdgpu_waves_per_eu(kSampleWaves))) void sample_compact_kernel(DScene s, ph_camera_view cam, int w, int h, uint32_t frame, uint32_t seed,
                                                                      PathOpts opt, float* color, float* albedo, float* emission, float* depth,
                                                                      uint32_t* normal, int* material) {
-    __shared__ int lds[kMegaDepth * kPixelBlock];
+    using Shape = PathStack<kPixelBlock, Wide>;
+    __shared__ int lds[Shape::kWords];
     const int tid = threadIdx.y * kBX + threadIdx.x;
-    SpillArea<kMegaDepth> spill;
-    LaneStack<kMegaDepth> stack{lds + tid, kPixelBlock, spill.v};
+    typename Shape::Spill spill;
+    auto stack = Shape::make(lds, tid, spill);
     const int x = blockIdx.x * kBX + threadIdx.x, y = blockIdx.y * kBY + threadIdx.y;
     if (x >= w || y >= h) return;
     const int i = y * w + x;
     PrimaryOut p{mk3(0), 0.0f, mk3(0), -1, mk3(1), mk3(0)};
-    f3 L = pixel_sample<LaneStack<kMegaDepth>, false>(s, cam, x, y, w, h, frame, seed, opt, &p, stack, nullptr);
+    f3 L = pixel_sample<typename Shape::Stack, false>(s, cam, x, y, w, h, frame, seed, opt, &p, stack, nullptr);
     color[3 * i] = L.x;
     color[3 * i + 1] = L.y;
     color[3 * i + 2] = L.z;
@@ -184,6 +190,18 @@ PH_DEV void trace_one(const DScene& s, const ph_ray* rays, int i, bool anyhit_fl
     (void)anyhit_flag;
 }
 
+// A wave's share of a ray buffer, its lanes refilled as they become free (trace_stream).
+template <bool AnyHit, class Walk, class Stack>
+PH_DEV void trace_rays(const ph_ray* rays, int n, int refill, const TraceScene& ts, Stack& stack, Walk& walk, ph_hit* hits) {
+    trace_stream<AnyHit>(
+        n, 1, refill, ts, stack, walk, [](int i) { return i; },
+        [&](int i, TraceScene&, auto& w) {
+            const float* r = reinterpret_cast<const float*>(rays + i);
+            w.start(mk3(r[0], r[1], r[2]), mk3(r[3], r[4], r[5]), r[6]);
+        },
+        [&](int i, const TraceScene&, const auto& w) { reinterpret_cast<float4*>(hits)[i] = make_float4(w.hit.t, __int_as_float(w.hit.tri), w.hit.u, w.hit.v); });
+}
+
 template <bool V>
 struct Tag {
     static constexpr bool value = V;
@@ -202,23 +220,30 @@ __global__ __launch_bounds__(Block) void trace_kernel(DScene s, const ph_ray* ra
         ts.top = top_nodes;
         ts.top_n = min(lds_nodes, s.top_nodes);
         stage_top_nodes(top_nodes, s.nodes, ts.top_n);
-        TraceCount c{0, 0, 0};
-        int idx = 0;  // this lane's ray
-        trace_stream<AnyHit, false>(
-            n, 1, 16, ts, stack, c,
-            [&](int i, TraceScene&, Walker& w, HitRec& hit) {
-                idx = i;
-                const float* r = reinterpret_cast<const float*>(rays + i);
-                w = walker(mk3(r[0], r[1], r[2]), mk3(r[3], r[4], r[5]), r[6]);
-                hit = HitRec{kInf, -1, 0.0f, 0.0f};
-            },
-            [&](const TraceScene&, const Walker&, const HitRec& hit) {
-                reinterpret_cast<float4*>(hits)[idx] = make_float4(hit.t, __int_as_float(hit.tri), hit.u, hit.v);
-            });
+        BinaryWalk<AnyHit, false> walk{};
+        trace_rays<AnyHit>(rays, n, 16, ts, stack, walk, hits);
     } else {
         const int i = blockIdx.x * Block + threadIdx.x;
         if (i < n) trace_one(s, rays, i, AnyHit, hits, counts, stack, Tag<Count>{}, Tag<AnyHit>{});
     }
+}
+
+// Closest hits over the wide nodes, a ray per lane: with rays in the caller's order a wave's rays end together, and
+// blocks that each take one ray per lane ran as fast as a fixed grid with refilled lanes (4,194,304 camera rays into
+// 262,144 triangles: 0.48 ms, against 0.49; over the binary nodes 0.99).
+constexpr int kRayBlock = 128;
+
+__global__ __launch_bounds__(kRayBlock) __attribute__((amdgpu_waves_per_eu(8))) void trace_wide_kernel(DScene s, const ph_ray* rays, int n, ph_hit* hits) {
+    using Shape = StackShape<kRayBlock, kWideLdsDepth, true>;
+    __shared__ int lds[Shape::kWords];
+    typename Shape::Spill spill;
+    auto stack = Shape::make(lds, threadIdx.x, spill);
+    const int i = blockIdx.x * kRayBlock + threadIdx.x;
+    if (i >= n) return;
+    const float* r = reinterpret_cast<const float*>(rays + i);
+    HitRec hit;
+    traverse_wide<false, false>(trace_scene(s), mk3(r[0], r[1], r[2]), mk3(r[3], r[4], r[5]), r[6], hit, stack);
+    reinterpret_cast<float4*>(hits)[i] = make_float4(hit.t, __int_as_float(hit.tri), hit.u, hit.v);
 }
 
 template <int Block, int Depth>
@@ -253,14 +278,14 @@ void trace_shape(hipStream_t st, const DScene& s, const ph_ray* rays, int n, boo
 void launch_render(hipStream_t st, const DScene& s, const ph_camera_view& cam, int w, int h, uint32_t frame0, int spp, uint32_t seed, const PathOpts& opt,
                    float4* accum, float4* albedo, float4* nd) {
     dim3 block(kBX, kBY), grid((w + kBX - 1) / kBX, (h + kBY - 1) / kBY);
-    hipLaunchKernelGGL(render_kernel, grid, block, 0, st, s, cam, w, h, frame0, spp, seed, opt, accum, albedo, nd);
+    hipLaunchKernelGGL(s.wide ? render_kernel<true> : render_kernel<false>, grid, block, 0, st, s, cam, w, h, frame0, spp, seed, opt, accum, albedo, nd);
     PH_CHECK(hipGetLastError());
 }
 
 void launch_sample(hipStream_t st, const DScene& s, const ph_camera_view& cam, int w, int h, uint32_t frame, uint32_t seed, const PathOpts& opt,
                    float4* color, float4* albedo, float4* nd, float4* position, float4* emission) {
     dim3 block(kBX, kBY), grid((w + kBX - 1) / kBX, (h + kBY - 1) / kBY);
-    hipLaunchKernelGGL(sample_kernel, grid, block, 0, st, s, cam, w, h, frame, seed, opt, color, albedo, nd, position, emission);
+    hipLaunchKernelGGL(s.wide ? sample_kernel<true> : sample_kernel<false>, grid, block, 0, st, s, cam, w, h, frame, seed, opt, color, albedo, nd, position, emission);
     PH_CHECK(hipGetLastError());
 }
 
@@ -273,7 +298,7 @@ void build_cdf_guides(hipStream_t st, const float* cdf, int rows, int n, size_t 
 void launch_sample_compact(hipStream_t st, const DScene& s, const ph_camera_view& cam, int w, int h, uint32_t frame, uint32_t seed, const PathOpts& opt,
                            const ph_compact_gbuffer& out) {
     dim3 block(kBX, kBY), grid((w + kBX - 1) / kBX, (h + kBY - 1) / kBY);
-    hipLaunchKernelGGL(sample_compact_kernel, grid, block, 0, st, s, cam, w, h, frame, seed, opt, static_cast<float*>(out.color_dev),
+    hipLaunchKernelGGL(s.wide ? sample_compact_kernel<true> : sample_compact_kernel<false>, grid, block, 0, st, s, cam, w, h, frame, seed, opt, static_cast<float*>(out.color_dev),
                        static_cast<float*>(out.albedo_dev), static_cast<float*>(out.emission_dev), static_cast<float*>(out.depth_dev),
                        static_cast<uint32_t*>(out.normal_dev), static_cast<int*>(out.material_dev));
     PH_CHECK(hipGetLastError());
@@ -289,6 +314,12 @@ void launch_display(hipStream_t st, const DisplayParams& p, const float4* accum,
                     const float4* variance, const float* heat, uint32_t* out) {
     dim3 block(kBX, kBY), grid((p.w + kBX - 1) / kBX, (p.h + kBY - 1) / kBY);
     hipLaunchKernelGGL(display_kernel, grid, block, 0, st, p, accum, denoised, albedo, nd, variance, heat, out);
+    PH_CHECK(hipGetLastError());
+}
+
+void launch_trace_wide(hipStream_t st, const DScene& s, const ph_ray* rays, int n, ph_hit* hits) {
+    if (n <= 0) return;
+    hipLaunchKernelGGL(trace_wide_kernel, dim3((n + kRayBlock - 1) / kRayBlock), dim3(kRayBlock), 0, st, s, rays, n, hits);
     PH_CHECK(hipGetLastError());
 }
 

@@ -521,74 +521,77 @@ __global__ __launch_bounds__(kCompactThreads) void compact_scatter_kernel(const 
     }
 }
 
+// The walk of a traversal kernel: over the wide nodes, or over the binary ones (counting kernels, staged top
+// nodes, scenes outside the wide nodes' limits).
+template <bool AnyHit, bool Count, bool Wide>
+using TraceWalk = std::conditional_t<Wide, WideWalk<AnyHit, !AnyHit>, BinaryWalk<AnyHit, Count>>;
+
 // Traversal of a queue of slots (trace_stream). One job: every lane shares the scene, whose traversal
-// arrays sit in scalar registers and whose top `lds_nodes` nodes the block stages in LDS. Serving: each
-// lane reads its slot's scene.
-template <bool AnyHit, bool Count, bool Multi, class Stack, class Load, class Finish>
+// arrays sit in scalar registers and whose top `lds_nodes` binary nodes the block stages in LDS. Serving:
+// each lane reads its slot's scene.
+template <bool AnyHit, bool Multi, class Walk, class Stack, class Load, class Finish>
 PH_DEV void trace_queue(const Work& work, const State& st, const int* queue, int n, int parts, int refill, int lds_nodes, float4* top, Stack& stack,
-                        TraceCount& cnt, Load load, Finish finish) {
+                        Walk& walk, Load load, Finish finish) {
     TraceScene ts0{};
     if (!Multi) {
         const JobParams j0 = single_job<false>(work);
-        ts0 = TraceScene{uniform_ptr(j0.scene.nodes), uniform_ptr(j0.scene.tris), &work.jobs[0].scene, top, min(lds_nodes, j0.scene.top_nodes)};
-        stage_top_nodes(top, ts0.nodes, ts0.top_n);
+        ts0 = TraceScene{uniform_ptr(j0.scene.nodes), uniform_ptr(j0.scene.tris), &work.jobs[0].scene, top, min(lds_nodes, j0.scene.top_nodes),
+                         uniform_ptr(j0.scene.wide)};
+        if constexpr (!Walk::kSecond) stage_top_nodes(top, ts0.nodes, ts0.top_n);
     }
-    int slot = 0, entry = 0;
-    trace_stream<AnyHit, Count>(
-        n, parts, refill, ts0, stack, cnt,
-        [&](int i, TraceScene& ts, Walker& w, HitRec& hit) {
-            slot = queue[i];
-            if (Multi) {
-                entry = st.job[slot];
-                ts = trace_scene(work.jobs[entry].scene);
-            }
-            load(slot, w, hit);
+    trace_stream<AnyHit>(
+        n, parts, refill, ts0, stack, walk, [&](int i) { return queue[i]; },
+        [&](int slot, TraceScene& ts, auto& w) {
+            if (Multi) ts = trace_scene(work.jobs[st.job[slot]].scene);
+            load(slot, w);
         },
-        [&](const TraceScene& ts, const Walker& w, const HitRec& hit) { finish(slot, entry, ts, w, hit); });
+        finish);
 }
 
-template <int Block, int Depth, bool Count, bool Multi>
-__global__ __launch_bounds__(Block) void extend_kernel(Work work, State st, int* counters, int sort, int refill, int lds_nodes, TraceTotals* totals) {
-    __shared__ int lds[Depth * Block];
+template <int Block, int Depth, bool Count, bool Multi, bool Wide>
+__global__ __launch_bounds__(Block) __attribute__((amdgpu_waves_per_eu(Wide ? 8 : 1))) void extend_kernel(Work work, State st, int* counters, int sort, int refill,
+                                                                                                            int lds_nodes, TraceTotals* totals) {
+    using Shape = StackShape<Block, Depth, Wide>;
+    __shared__ int lds[Shape::kWords];
     extern __shared__ float4 top_nodes[];
-    SpillArea<Depth> spill;
-    LaneStack<Depth> stack{lds + threadIdx.x, Block, spill.v};
-    TraceCount cnt{0, 0, 0};
-    trace_queue<false, Count, Multi>(
-        work, st, st.q_ext, counters[C_EXT], counters[C_PARTS], refill, lds_nodes, top_nodes, stack, cnt,
-        [&](int slot, Walker& w, HitRec& hit) {
+    typename Shape::Spill spill;
+    auto stack = Shape::make(lds, threadIdx.x, spill);
+    TraceWalk<false, Count, Wide> walk{};
+    trace_queue<false, Multi>(
+        work, st, st.q_ext, counters[C_EXT], counters[C_PARTS], refill, lds_nodes, top_nodes, stack, walk,
+        [&](int slot, auto& w) {
             const float4 o4 = ld_stream(st.ro + slot), d4 = ld_stream(st.rd + slot);
-            w = walker(xyz(o4), xyz(d4), kInf);
-            hit = HitRec{kInf, -1, 0.0f, 0.0f};
+            w.start(xyz(o4), xyz(d4), kInf);
         },
-        [&](int slot, int entry, const TraceScene& ts, const Walker&, const HitRec& hit) {
-            st_stream(st.hit + slot, make_float4(hit.t, __int_as_float(hit.tri), hit.u, hit.v));
+        [&](int slot, const TraceScene& ts, const auto& w) {
+            st_stream(st.hit + slot, make_float4(w.hit.t, __int_as_float(w.hit.tri), w.hit.u, w.hit.v));
             uint8_t next = S_MISS;
-            if (hit.tri >= 0) {
-                const int* cls = work.jobs[entry].mat_class;
-                next = uint8_t(S_CLASS + (sort ? ldg(cls + __float_as_int(ldg(ts.tris + 3 * hit.tri).w)) : kClasses - 1));
+            if (w.hit.tri >= 0) {
+                const int* cls = work.jobs[Multi ? st.job[slot] : 0].mat_class;
+                next = uint8_t(S_CLASS + (sort ? ldg(cls + w.material_of(ts)) : kClasses - 1));
             }
             st.stage[slot] = next;
         });
-    if (Count) flush_counts(cnt, totals);
+    if constexpr (Count) flush_counts(walk.cnt, totals);
 }
 
-template <int Block, int Depth, bool Count, bool Multi>
-__global__ __launch_bounds__(Block) void shadow_kernel(Work work, State st, int* counters, int refill, int lds_nodes, TraceTotals* totals) {
-    __shared__ int lds[Depth * Block];
+template <int Block, int Depth, bool Count, bool Multi, bool Wide>
+__global__ __launch_bounds__(Block) __attribute__((amdgpu_waves_per_eu(Wide ? 8 : 1))) void shadow_kernel(Work work, State st, int* counters, int refill,
+                                                                                                            int lds_nodes, TraceTotals* totals) {
+    using Shape = StackShape<Block, Depth, Wide>;
+    __shared__ int lds[Shape::kWords];
     extern __shared__ float4 top_nodes[];
-    SpillArea<Depth> spill;
-    LaneStack<Depth> stack{lds + threadIdx.x, Block, spill.v};
-    TraceCount cnt{0, 0, 0};
-    trace_queue<true, Count, Multi>(
-        work, st, st.q_shadow, counters[C_SHADOW], counters[C_PARTS], refill, lds_nodes, top_nodes, stack, cnt,
-        [&](int slot, Walker& w, HitRec& hit) {
+    typename Shape::Spill spill;
+    auto stack = Shape::make(lds, threadIdx.x, spill);
+    TraceWalk<true, Count, Wide> walk{};
+    trace_queue<true, Multi>(
+        work, st, st.q_shadow, counters[C_SHADOW], counters[C_PARTS], refill, lds_nodes, top_nodes, stack, walk,
+        [&](int slot, auto& w) {
             const float4 o4 = ld_stream(st.so + slot), d4 = ld_stream(st.sd + slot);
-            w = walker(xyz(o4), xyz(d4), o4.w);
-            hit = HitRec{kInf, -1, 0.0f, 0.0f};
+            w.start(xyz(o4), xyz(d4), o4.w);
         },
-        [&](int slot, int, const TraceScene&, const Walker& w, const HitRec&) {
-            if (w.found) return;
+        [&](int slot, const TraceScene&, const auto& w) {
+            if (w.hit.tri >= 0) return;
             const float4 c = ld_stream(st.sc + slot);
             float4 L = ld_stream(st.L + slot);
             L.x += c.x;
@@ -596,7 +599,7 @@ __global__ __launch_bounds__(Block) void shadow_kernel(Work work, State st, int*
             L.z += c.z;
             st_stream(st.L + slot, L);
         });
-    if (Count) flush_counts(cnt, totals);
+    if constexpr (Count) flush_counts(walk.cnt, totals);
 }
 
 template <bool Multi>
@@ -801,7 +804,7 @@ __global__ void advance_items_kernel(unsigned long long* items, const int* count
 // the per-pixel kernel runs a pixel: the path from its pending extension ray (trace_path_from, same
 // vertices, same draws), then the item's remaining samples, accumulated as regen_kernel accumulates
 // them. The queue is then cleared (finish_clear_kernel) and the rest of the iteration finds no work.
-constexpr int kFinishBlock = 128, kFinishDepth = 32;
+constexpr int kFinishBlock = 128;
 
 PH_DEV bool finish_now(const int* counters, const unsigned long long* items, int limit) {
     const int n = counters[C_EXT];
@@ -811,12 +814,14 @@ PH_DEV bool finish_now(const int* counters, const unsigned long long* items, int
 // tally: [0] extension rays, [1] shadow rays, [2] paths finished. Lanes take queue entries as they become
 // free (one atomic per wave and refill, on C_FINISH), and run one sample per loop turn, so a lane whose
 // item ends takes the next entry instead of idling while its wave finishes longer paths.
+template <bool Wide>
 __global__ __launch_bounds__(kFinishBlock) __attribute__((amdgpu_waves_per_eu(4))) void finish_kernel(Work work, State st, int* counters, int limit,
                                                                                                         unsigned long long* rays) {
     if (!finish_now(counters, work.items, limit)) return;
-    __shared__ int lds[kFinishDepth * kFinishBlock];
-    SpillArea<kFinishDepth> spill;
-    LaneStack<kFinishDepth> stack{lds + threadIdx.x, kFinishBlock, spill.v};
+    using Shape = PathStack<kFinishBlock, Wide>;
+    __shared__ int lds[Shape::kWords];
+    typename Shape::Spill spill;
+    auto stack = Shape::make(lds, threadIdx.x, spill);
     const int n = counters[C_EXT];
     const JobParams jp = single_job<false>(work);
     const bool parts = jp.split > 1;
@@ -855,7 +860,7 @@ __global__ __launch_bounds__(kFinishBlock) __attribute__((amdgpu_waves_per_eu(4)
                 const bool first = ps.depth == 0 && k == 0 && jp.albedo;
                 PrimaryOut prim{mk3(0), 0.0f, mk3(0), -1, mk3(1), mk3(0)};
                 Pcg rng = slot_rng(st, slot, pixel);
-                L = trace_path_from<LaneStack<kFinishDepth>, false>(jp.scene, xyz(o4), xyz(d4), rng, jp.opt, ps, first ? &prim : nullptr, stack,
+                L = trace_path_from<typename Shape::Stack, false>(jp.scene, xyz(o4), xyz(d4), rng, jp.opt, ps, first ? &prim : nullptr, stack,
                                                                     nullptr, &tally);
                 if (first) {
                     jp.albedo[pixel] = make_float4(prim.albedo.x, prim.albedo.y, prim.albedo.z, 1.0f);
@@ -863,7 +868,7 @@ __global__ __launch_bounds__(kFinishBlock) __attribute__((amdgpu_waves_per_eu(4)
                 }
                 resumed = true;
             } else {
-                L = pixel_sample<LaneStack<kFinishDepth>, false>(jp.scene, jp.camera, pixel % jp.width, pixel / jp.width, jp.width, jp.height,
+                L = pixel_sample<typename Shape::Stack, false>(jp.scene, jp.camera, pixel % jp.width, pixel / jp.width, jp.width, jp.height,
                                                                  jp.frame0 + uint32_t(k), jp.seed, jp.opt, nullptr, stack, nullptr, &tally);
             }
             if (!finite3(L) || L.x < 0 || L.y < 0 || L.z < 0) L = mk3(0);
@@ -928,26 +933,30 @@ int device_cus() {
     return cus;
 }
 
-using TraceLaunch = void (*)(hipStream_t, int, Work, State, int*, int, int, int, TraceTotals*, bool);
+using TraceLaunch = void (*)(hipStream_t, int, Work, State, int*, int, int, int, TraceTotals*, bool, bool);
 
 template <int Block, int Depth, bool Multi>
-void launch_extend(hipStream_t st, int grid, Work w, State s, int* counters, int sort, int refill, int lds_nodes, TraceTotals* tot, bool count) {
-    const size_t lds = Multi ? 0 : size_t(lds_nodes) * 64;
+void launch_extend(hipStream_t st, int grid, Work w, State s, int* counters, int sort, int refill, int lds_nodes, TraceTotals* tot, bool count, bool wide) {
+    const int top = Multi ? 0 : lds_nodes;
+    const size_t lds = size_t(top) * 64;
     if (count)
-        hipLaunchKernelGGL((extend_kernel<Block, Depth, true, Multi>), dim3(grid), dim3(Block), lds, st, w, s, counters, sort, refill, Multi ? 0 : lds_nodes,
-                           tot);
+        hipLaunchKernelGGL((extend_kernel<Block, Depth, true, Multi, false>), dim3(grid), dim3(Block), lds, st, w, s, counters, sort, refill, top, tot);
+    else if (!wide || top)
+        hipLaunchKernelGGL((extend_kernel<Block, Depth, false, Multi, false>), dim3(grid), dim3(Block), lds, st, w, s, counters, sort, refill, top, tot);
     else
-        hipLaunchKernelGGL((extend_kernel<Block, Depth, false, Multi>), dim3(grid), dim3(Block), lds, st, w, s, counters, sort, refill, Multi ? 0 : lds_nodes,
-                           tot);
+        hipLaunchKernelGGL((extend_kernel<Block, kWideLdsDepth, false, Multi, true>), dim3(grid), dim3(Block), 0, st, w, s, counters, sort, refill, 0, tot);
 }
 
 template <int Block, int Depth, bool Multi>
-void launch_shadow(hipStream_t st, int grid, Work w, State s, int* counters, int, int refill, int lds_nodes, TraceTotals* tot, bool count) {
-    const size_t lds = Multi ? 0 : size_t(lds_nodes) * 64;
+void launch_shadow(hipStream_t st, int grid, Work w, State s, int* counters, int, int refill, int lds_nodes, TraceTotals* tot, bool count, bool wide) {
+    const int top = Multi ? 0 : lds_nodes;
+    const size_t lds = size_t(top) * 64;
     if (count)
-        hipLaunchKernelGGL((shadow_kernel<Block, Depth, true, Multi>), dim3(grid), dim3(Block), lds, st, w, s, counters, refill, Multi ? 0 : lds_nodes, tot);
+        hipLaunchKernelGGL((shadow_kernel<Block, Depth, true, Multi, false>), dim3(grid), dim3(Block), lds, st, w, s, counters, refill, top, tot);
+    else if (!wide || top)
+        hipLaunchKernelGGL((shadow_kernel<Block, Depth, false, Multi, false>), dim3(grid), dim3(Block), lds, st, w, s, counters, refill, top, tot);
     else
-        hipLaunchKernelGGL((shadow_kernel<Block, Depth, false, Multi>), dim3(grid), dim3(Block), lds, st, w, s, counters, refill, Multi ? 0 : lds_nodes, tot);
+        hipLaunchKernelGGL((shadow_kernel<Block, kWideLdsDepth, false, Multi, true>), dim3(grid), dim3(Block), 0, st, w, s, counters, refill, 0, tot);
 }
 
 struct ShapeFns {
@@ -1023,12 +1032,14 @@ struct WavefrontEngine::Impl {
     unsigned long long* host_stage = nullptr;  // staging of item counts for upload
     std::vector<hipEvent_t> events;
     hipGraphExec_t graph_exec = nullptr;
-    std::tuple<int, int, int, int, int, bool> graph_key{};
+    std::tuple<int, int, int, int, int, bool, bool> graph_key{};
+    bool wide = false;  // every scene in work has wide nodes
     std::map<std::tuple<const void*, int, int, int, int>, ph_wavefront_config> tuned;
     // Serving bookkeeping (host side).
     bool serving = false;
     std::vector<bool> entry_used;
     std::vector<int> entry_pixels;
+    std::vector<bool> entry_wide;
     // A queued pass: its unstarted items are [next, pixels) of the job's pixel order. While laid out,
     // its items occupy the segments (first, length) of the item index space, in pixel order: one
     // segment for a contiguous layout, one per round for a round-robin one.
@@ -1062,6 +1073,7 @@ struct WavefrontEngine::Impl {
         cus = device_cus();
         entry_used.assign(kMaxJobs, false);
         entry_pixels.assign(kMaxJobs, 0);
+        entry_wide.assign(kMaxJobs, false);
     }
     ~Impl() {
         drop_graph();
@@ -1150,18 +1162,23 @@ struct WavefrontEngine::Impl {
     // One bounce. Event pairs bracket the traversal launches when timing.
     template <bool Multi>
     void iteration(hipStream_t st, const ShapeFns& fns, bool count, hipEvent_t* ev) {
-        const int tgrid = cus * std::max(1, cfg.blocks_per_cu);
+        // Traversal: what fits the chip at once, or over the wide nodes four times that. The shares of a wave cost very
+        // differently, and blocks that start as others end even them out (1080p, 64 samples, 1M triangles: 79.0 ms,
+        // 83.0 with one round of blocks, 81.1 with two). Never more lanes than slots: a queue holds no more.
+        const auto blocks_for = [&](int most, int block) { return std::max(1, std::min(most, (slots + block - 1) / block)); };
+        const bool over_wide = wide && !count && (Multi || cfg.lds_nodes == 0);
+        const int tgrid = blocks_for(cus * std::max(1, cfg.blocks_per_cu) * (over_wide ? 4 : 1), cfg.block);
         // Shading: 4 blocks of 256 threads per CU. The shading kernels use 232 VGPRs (2 waves per SIMD), so
         // half of the blocks start as the others finish their share. Compiling them for 6 or 8 waves (with a
         // grid to match) spills and was slower: 940 and 897 against 995 Msamples/s.
-        const int sgrid = cus * 4;
+        const int sgrid = blocks_for(cus * 4, 256);
         const State s = state();
         const Work w = work();
         int* cnt = counters.ptr;
         hipLaunchKernelGGL(bookkeep_kernel, dim3(1), dim3(64), 0, st, cnt, ray_totals.ptr);
         if (ev) PH_CHECK(hipEventRecord(ev[0], st));
         const int refill = std::clamp(cfg.refill_lanes, 1, 64);
-        fns.extend(st, tgrid, w, s, cnt, cfg.sort_materials ? 1 : 0, refill, cfg.lds_nodes, totals.ptr, count);
+        fns.extend(st, tgrid, w, s, cnt, cfg.sort_materials ? 1 : 0, refill, cfg.lds_nodes, totals.ptr, count, wide);
         if (ev) PH_CHECK(hipEventRecord(ev[1], st));
         compact<K_HIT, Multi>(st, s);
         hipLaunchKernelGGL(miss_kernel<Multi>, dim3(sgrid), dim3(256), 0, st, w, s, cnt);
@@ -1172,14 +1189,15 @@ struct WavefrontEngine::Impl {
         hipLaunchKernelGGL((shade_kernel<7, Multi>), dim3(sgrid), dim3(256), 0, st, w, s, cnt, 3, bins);
         compact<K_DONE, Multi>(st, s);
         if (ev) PH_CHECK(hipEventRecord(ev[2], st));
-        fns.shadow(st, tgrid, w, s, cnt, 0, refill, cfg.lds_nodes, totals.ptr + 1, count);
+        fns.shadow(st, tgrid, w, s, cnt, 0, refill, cfg.lds_nodes, totals.ptr + 1, count, wide);
         if (ev) PH_CHECK(hipEventRecord(ev[3], st));
         hipLaunchKernelGGL(regen_kernel<Multi>, dim3(sgrid), dim3(256), 0, st, w, s, cnt);
         hipLaunchKernelGGL(advance_items_kernel, dim3(1), dim3(64), 0, st, items.ptr, cnt);
         compact<K_EXT, Multi>(st, s);
         const int finish_limit = int(int64_t(slots) * std::clamp(cfg.finish_percent, 0, 100) / 100);
         if (!Multi && finish_limit > 0) {
-            hipLaunchKernelGGL(finish_kernel, dim3(cus * 8), dim3(kFinishBlock), 0, st, w, s, cnt, finish_limit, ray_totals.ptr + 2);
+            hipLaunchKernelGGL(wide ? finish_kernel<true> : finish_kernel<false>, dim3(cus * 8), dim3(kFinishBlock), 0, st, w, s, cnt, finish_limit,
+                               ray_totals.ptr + 2);
             hipLaunchKernelGGL(finish_clear_kernel, dim3(1), dim3(64), 0, st, cnt, items.ptr, finish_limit);
         }
         PH_CHECK(hipGetLastError());
@@ -1198,7 +1216,7 @@ struct WavefrontEngine::Impl {
         const ShapeFns fns = shapes(multi);
         const bool graph = cfg.use_graph != 0 && !counting;
         if (graph) {
-            auto key = std::make_tuple(cfg.block, cfg.stack_depth, cfg.blocks_per_cu, G, slots, multi);
+            auto key = std::make_tuple(cfg.block, cfg.stack_depth, cfg.blocks_per_cu, G, slots, multi, wide);
             if (!graph_exec || key != graph_key) {
                 drop_graph();
                 hipGraph_t g = nullptr;
@@ -1311,6 +1329,7 @@ void WavefrontEngine::render(hipStream_t st, const WavefrontJob& job, bool count
     // Paths in flight: one per pixel up to a cap of 4M slots (~900 MB of state), never more than items.
     const int slots = int(std::min<int64_t>(m.cfg.path_slots > 0 ? m.cfg.path_slots : std::min(pixels, 1 << 22), items));
     m.ensure_slots(slots);
+    m.wide = job.scene.wide != nullptr;
     if (!job.mat_class) {
         std::vector<int> cls = material_classes(job.scene, st);
         m.mat_class.upload(cls.data(), cls.size(), st);
@@ -1519,6 +1538,7 @@ int WavefrontEngine::serve_admit(hipStream_t st, const WavefrontJob& job) {
     PH_CHECK(hipMemsetAsync(m.job_done.ptr + entry, 0, sizeof(int), st));
     m.host_done[entry] = 0;
     m.entry_used[size_t(entry)] = true;
+    m.entry_wide[size_t(entry)] = job.scene.wide != nullptr;
     m.entry_pixels[size_t(entry)] = job.width * job.height * job.split;
     return entry;
 }
@@ -1616,6 +1636,9 @@ void WavefrontEngine::serve_run(hipStream_t st, int iterations) {
     }
     m.passes.swap(keep);
     m.chunks_dirty = false;
+    m.wide = true;
+    for (int e = 0; e < kMaxJobs; e++)
+        if (m.entry_used[size_t(e)] && !m.entry_wide[size_t(e)]) m.wide = false;
     m.run_batch(st, std::max(1, iterations), true, false);
     PH_CHECK(hipMemcpyAsync(m.host_done, m.job_done.ptr, kMaxJobs * sizeof(int), hipMemcpyDeviceToHost, st));
     PH_CHECK(hipStreamSynchronize(st));

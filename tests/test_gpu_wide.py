@@ -1,0 +1,128 @@
+"""The walk over the four-wide nodes against the walk over the binary ones, bit for bit: a traced ray buffer
+goes over the wide nodes, a counted one over the binary ones, and the wavefront engine takes the binary nodes
+when their top is staged in LDS. Scenes where ties, flat boxes, rounding or the wide format's limits decide."""
+import numpy as np
+import pytest
+
+from photon_amd import gpu, host
+from photon_amd.types import RAY_DTYPE, Material, RenderSettings
+
+from gpu_util import trace_on_gpu, uploaded
+
+pytestmark = pytest.mark.gpu
+
+
+def _mesh(scale=1.0, offset=0.0, twice=False, n=900, flat=False, max_leaf=0, seed=3):
+    """Random small triangles, or a floor of axis-aligned ones; `twice`: every triangle again, in a second mesh."""
+    rng = np.random.default_rng(seed)
+    if flat:
+        k = int(np.sqrt(n / 2))
+        x, z = np.meshgrid(np.arange(k), np.arange(k))
+        corner = np.stack([x, np.zeros_like(x), z], -1).reshape(-1, 1, 3).astype(np.float64)
+        quad = np.array([[0, 0, 0], [1, 0, 0], [1, 0, 1], [0, 0, 0], [1, 0, 1], [0, 0, 1]], float)
+        p = (corner + quad).reshape(-1, 3) / k * 2 - 1
+    else:
+        p = (rng.uniform(-1, 1, (n, 1, 3)) + rng.normal(0, 0.08, (n, 3, 3))).reshape(-1, 3)
+    p = (p * scale + offset).astype(np.float32)
+    s = host.Scene()
+    for _ in range(2 if twice else 1):
+        s.add_mesh(p, np.arange(len(p), dtype=np.int32), s.add_material(Material.default()))
+    return s.build(max_leaf=max_leaf, traversal_cost=1e9 if max_leaf > 32 else 0.0), p
+
+
+def _rays(points, n, seed):
+    """Rays between points near the vertices `points`, many of them exactly through vertices and edges, along axes,
+    from far away, and with upper limits that cut hits off; a few that are not finite."""
+    rng = np.random.default_rng(seed)
+    lo, hi = points.min(0), points.max(0)
+    ext = np.maximum(hi - lo, 1e-6 * np.abs(hi))
+    ext = np.maximum(ext, ext.max() * 1e-3)
+    tri = points[: len(points) // 3 * 3].reshape(-1, 3, 3)
+    t = tri[rng.integers(len(tri), size=n)].astype(np.float64)
+    bary = rng.dirichlet(np.ones(3), n)
+    edge = rng.random(n) < 0.25
+    bary[edge, 0] = 0
+    vertex = rng.random(n) < 0.15
+    bary[vertex] = [0, 1, 0]
+    target = (t * (bary / bary.sum(1, keepdims=True))[..., None]).sum(1)
+    o = lo + ext * rng.uniform(-1.0, 2.0, (n, 3))
+    far = rng.random(n) < 0.2
+    o[far] = target[far] + (o - target)[far] * 10.0 ** rng.uniform(0, 6, (far.sum(), 1))
+    on = rng.random(n) < 0.1
+    o[on] = t[on, 0]
+    d = target - o
+    d /= np.maximum(np.linalg.norm(d, axis=1, keepdims=True), 1e-30)
+    axis = rng.random(n) < 0.2
+    k = rng.integers(3, size=n)
+    unit = np.eye(3)[k] * rng.choice([-1.0, 1.0], n)[:, None]
+    o[axis] = target[axis] - unit[axis] * ext[k[axis], None]
+    d[axis] = unit[axis]
+    d[rng.random(n) < 0.03] *= -0.0
+    r = np.zeros(n, RAY_DTYPE)
+    r["o"], r["d"], r["tmax"] = o, d, 1e30
+    cut = rng.random(n) < 0.2
+    r["tmax"][cut] = (ext.max() * 10.0 ** rng.uniform(-3, 1, cut.sum())).astype(np.float32)
+    r["tmax"][:6] = [0.0, -1.0, np.nan, np.inf, 3e38, 1e-30]
+    r["o"][6:9, 0] = [np.nan, 1e16, -np.inf]
+    r["d"][9:13, 1] = [np.nan, 1e16, np.inf, 1e-25]
+    return r
+
+
+CASES = {
+    "random": dict(),
+    "twice": dict(twice=True, n=300),
+    "floor": dict(flat=True),
+    "floor-twice": dict(flat=True, twice=True, n=400),
+    "tiny": dict(scale=1e-6),
+    "small-far": dict(scale=1e-2, offset=1e3),
+    "large": dict(scale=1e6),
+    "beyond-limits": dict(scale=1e16, n=60),
+    "large-leaves": dict(n=200, max_leaf=200),
+    "one": dict(n=1),
+    "five": dict(n=5),
+}
+
+
+@pytest.mark.parametrize("name", sorted(CASES))
+def test_wide_hits_are_the_binary_hits(name):
+    scene, points = _mesh(**CASES[name])
+    r = uploaded(scene)
+    rays = _rays(points, 40001, seed=len(name))
+    want, _ = trace_on_gpu(r, rays, counts=True)
+    got = trace_on_gpu(r, rays)
+    # The bounds under rays at the tie threshold: limits set to a hit's own distance.
+    hit = want["tri"] >= 0
+    limited = rays.copy()
+    limited["tmax"][hit] = want["t"][hit] * np.where(np.arange(hit.sum()) % 2, np.float32(1), np.float32(1 + 2**-22))
+    want2, _ = trace_on_gpu(r, limited, counts=True)
+    got2 = trace_on_gpu(r, limited)
+    assert name in ("beyond-limits", "tiny") or hit.mean() > 0.1
+    assert got.tobytes() == want.tobytes()
+    assert got2.tobytes() == want2.tobytes()
+    r.close()
+
+
+@pytest.mark.parametrize("name", ["cornell-c1", "materials", "glass", "soup"])
+def test_wide_hits_on_scenes(name):
+    scene = host.Scene.spheres(24, box=20.0, alpha_fraction=0.3, seed=5).build() if name == "soup" else host.Scene.builtin(name).build()
+    r = uploaded(scene)
+    rays = host.camera_rays(scene.camera_view(1.0), 257, 251)
+    assert trace_on_gpu(r, rays).tobytes() == trace_on_gpu(r, rays, counts=True)[0].tobytes()
+    r.close()
+
+
+@pytest.mark.parametrize("w,h,spp,split", [(70, 45, 3, 1), (130, 67, 4, 4)])
+def test_wavefront_image_over_either_walk(w, h, spp, split):
+    """Also a second upload and a light update, which write the triangles again."""
+    scene = host.Scene.field(8, seed=2, env_width=64).build()
+    cam, rs = scene.camera_view(w / h), RenderSettings.make(w, h, max_depth=8, rr_depth=3, seed=9)
+    r = uploaded(scene, w, h, engine=gpu.ENGINE_WAVEFRONT)
+    images = []
+    for nodes in (0, 64, 0):
+        r.set_wavefront_config(block=64, stack_depth=8, path_slots=1000, lds_nodes=nodes, sample_split=split)
+        r.reset()
+        r.render(cam, rs, spp)
+        images.append(r.download_image())
+        r.update_lights(scene)
+    assert images[0].tobytes() == images[1].tobytes() == images[2].tobytes()
+    r.close()
