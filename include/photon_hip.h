@@ -52,7 +52,8 @@ typedef struct ph_gpu_info {
 typedef struct ph_wavefront_config {
     int32_t block;         /* threads per block of the traversal kernels: 64, 128, 256 */
     int32_t stack_depth;   /* LDS stack entries per lane: 8, 16, 24, 32, 64 (rest spills to scratch) */
-    int32_t path_slots;    /* paths in flight (0: one per pixel, capped by memory) */
+    int32_t path_slots;    /* paths in flight (0: one per pixel, capped by memory; with sample_split 1 as well, the render's
+                              size decides: chunks of whole samples, each sample a work item, with the same image) */
     int32_t blocks_per_cu; /* persistent grid: blocks per compute unit */
     int32_t sort_materials;/* shade in material-class queues */
     int32_t use_graph;     /* replay the bounce loop from a captured HIP graph */
@@ -61,7 +62,7 @@ typedef struct ph_wavefront_config {
     int32_t lds_nodes;     /* top BVH nodes (breadth-first) each traversal block stages in LDS */
     int32_t ray_bins;      /* trace camera rays, then continuing rays by direction octant (1), or all together (0) */
     int32_t xcd_parts;     /* 8: each XCD takes a contiguous eighth of every queue (L2 locality); 1: all waves interleave */
-    int32_t sample_split;  /* 1: a path slot runs all of a pixel's samples in order, and the accumulation is bit-identical
+    int32_t sample_split;  /* 1: all of a pixel's samples are added in order, and the accumulation is bit-identical
                               to the per-pixel kernel's (the reference's order). S > 1: each pixel's samples run as S
                               sub-streams of spp/S samples (S rounded down to a divisor of spp) that any slot may take,
                               into partial sums that are added to the accumulation in sub-stream order; deterministic,

@@ -69,6 +69,8 @@ public:
     int64_t serve_work_remaining() const;
 
 private:
+    void render_chunk(hipStream_t st, const WavefrontJob& job, int split, int64_t most, int G, bool counting, ph_render_stats& stats);
+    void render_direct(hipStream_t st, const WavefrontJob& job, ph_render_stats& stats);
     struct Impl;
     std::unique_ptr<Impl> impl_;
 };

@@ -896,6 +896,52 @@ __global__ void finish_clear_kernel(int* counters, const unsigned long long* ite
     if (threadIdx.x == 0 && finish_now(counters, items, limit)) counters[C_EXT] = 0;
 }
 
+// ---- small renders --------------------------------------------------------------------------------------
+// A render (or chunk of one) of few samples, a sample per lane: the per-pixel kernel's integrator, but all samples
+// of a pixel at once, neighbouring lanes running neighbouring samples of the same pixels. The bounce loop costs
+// such a render about 20 launches a bounce, most of them nearly empty. What bounds this kernel is the longest path
+// of each wave. Sums go to the sub-streams' partial sums (or the accumulation, with one sample).
+// rays: kDirectTallies pairs (extension, shadow), added up by the caller; one pair would serialize the waves.
+constexpr int kDirectBlock = 128, kDirectTallies = 64;
+
+template <bool Wide>
+__global__ __launch_bounds__(kDirectBlock) __attribute__((amdgpu_waves_per_eu(4))) void direct_kernel(JobParams jp, unsigned long long* rays) {
+    using Shape = PathStack<kDirectBlock, Wide>;
+    __shared__ int lds[Shape::kWords];
+    typename Shape::Spill spill;
+    auto stack = Shape::make(lds, threadIdx.x, spill);
+    RayTally tally{0, 0};
+    const int i = blockIdx.x * kDirectBlock + threadIdx.x;
+    if (i < jp.pixels * jp.split) {
+        const int part = int(uint32_t(i) % uint32_t(jp.split));
+        const int pixel = work_pixel(int(uint32_t(i) / uint32_t(jp.split)), jp.width, jp.height);
+        const bool first = part == 0 && jp.albedo;
+        PrimaryOut prim{mk3(0), 0.0f, mk3(0), -1, mk3(1), mk3(0)};
+        const f3 L = pixel_sample<typename Shape::Stack, false>(jp.scene, jp.camera, pixel % jp.width, pixel / jp.width, jp.width, jp.height,
+                                                                jp.frame0 + uint32_t(part), jp.seed, jp.opt, first ? &prim : nullptr, stack, nullptr, &tally);
+        float4* acc = jp.accum + size_t(pixel) * size_t(jp.split) + size_t(part);
+        float4 a = jp.split > 1 ? make_float4(0.0f, 0.0f, 0.0f, 0.0f) : *acc;
+        a.x += L.x;
+        a.y += L.y;
+        a.z += L.z;
+        const float l = lum(L);
+        a.w += l * l;
+        *acc = a;
+        if (first) {
+            jp.albedo[pixel] = make_float4(prim.albedo.x, prim.albedo.y, prim.albedo.z, 1.0f);
+            jp.nd[pixel] = make_float4(prim.normal.x, prim.normal.y, prim.normal.z, prim.depth);
+        }
+    }
+    const unsigned long long e = wave_sum(tally.ext), sh = wave_sum(tally.shadow);
+    if (lane_id() == 0) {
+        unsigned long long* r = rays + 2 * (blockIdx.x % kDirectTallies);
+        atomicAdd(r, e);
+        atomicAdd(r + 1, sh);
+    }
+}
+
+__global__ __launch_bounds__(2 * kDirectTallies) void clear_tallies_kernel(unsigned long long* rays) { rays[threadIdx.x] = 0; }
+
 // The end of a single render in sub-streams: adds the partial sums to the accumulation, sub-stream 0
 // first. The sums of a pixel are consecutive: a block stages those of kPartPixels pixels in LDS, kPartRun
 // of each at a time, with coalesced loads, and one lane per pixel and component adds them in order. The
@@ -1022,6 +1068,7 @@ struct WavefrontEngine::Impl {
     DevBuf<uint64_t> rng;
     DevBuf<float4> ro, rd, beta, L, hit, so, sd, sc;
     DevBuf<float4> part_sums;  // partial sums of a single render in sub-streams
+    DevBuf<unsigned long long> direct_rays;  // direct_kernel's tallies
     DevBuf<JobParams> jobs;
     DevBuf<TraceTotals> totals;             // [0] extension rays, [1] shadow rays
     DevBuf<unsigned long long> ray_totals;  // rays traced: [0] extension, [1] shadow; finish_kernel: [2] extension, [3] shadow, [4] paths
@@ -1030,6 +1077,7 @@ struct WavefrontEngine::Impl {
     int* host_sizes = nullptr;
     unsigned long long* host_items = nullptr;  // after a batch: next item, items queued
     unsigned long long* host_stage = nullptr;  // staging of item counts for upload
+    unsigned long long* host_direct = nullptr;  // direct_kernel's tallies
     std::vector<hipEvent_t> events;
     hipGraphExec_t graph_exec = nullptr;
     std::tuple<int, int, int, int, int, bool, bool> graph_key{};
@@ -1061,6 +1109,7 @@ struct WavefrontEngine::Impl {
         PH_CHECK(hipHostMalloc(reinterpret_cast<void**>(&host_sizes), 2 * sizeof(int), hipHostMallocDefault));
         PH_CHECK(hipHostMalloc(reinterpret_cast<void**>(&host_items), 2 * sizeof(unsigned long long), hipHostMallocDefault));
         PH_CHECK(hipHostMalloc(reinterpret_cast<void**>(&host_stage), 2 * sizeof(unsigned long long), hipHostMallocDefault));
+        PH_CHECK(hipHostMalloc(reinterpret_cast<void**>(&host_direct), 2 * kDirectTallies * sizeof(unsigned long long), hipHostMallocDefault));
         std::memset(host_items, 0, 2 * sizeof(unsigned long long));
         counters.allocate(C_COUNT);
         jobs.allocate(kMaxJobs);
@@ -1083,6 +1132,7 @@ struct WavefrontEngine::Impl {
         if (host_sizes) (void)hipHostFree(host_sizes);
         if (host_items) (void)hipHostFree(host_items);
         if (host_stage) (void)hipHostFree(host_stage);
+        if (host_direct) (void)hipHostFree(host_direct);
     }
 
     void drop_graph() {
@@ -1313,21 +1363,87 @@ void WavefrontEngine::set_config(const ph_wavefront_config& c) {
 
 ph_wavefront_config WavefrontEngine::config() const { return impl_->cfg; }
 
+// Launch rule of the default configuration (no path slots or sub-streams asked for): the render runs in chunks of
+// whole samples, every sample of a chunk its own work item. The partial sums are single samples, added in sample
+// order, so the image is the in-order one bit for bit, and a chunk lasts as long as its longest paths, not as long as
+// the pixel with the longest run of them. 853x479, 8 samples of the materials scene: 3.5 ms, 11.8 with one item a
+// pixel; the 1M-triangle field's geometry at 1080p x 64 about 61 ms, 110 before. kChunkItems bounds the partial sums
+// (1 GB) and kChunkSlots the paths' state (1.7 GB; at 4M slots the field takes 68 ms). Two bounces a graph: a bounce
+// that finds nothing costs 0.1 ms, a look at the queue 0.03. Chunks of at most kDirectItems samples run a sample per
+// lane: 64x64x4 Cornell box 0.32 ms (0.65 in bounces), 320x240x12 glass 1.56 (1.81), 640x360x4 materials 1.49 (2.1),
+// while 853x479x8 would take 4.4 against 3.5.
+constexpr int64_t kChunkItems = int64_t(1) << 26, kChunkSlots = int64_t(1) << 23, kDirectItems = int64_t(1) << 20;
+constexpr int kChunkGraph = 2;
+
 void WavefrontEngine::render(hipStream_t st, const WavefrontJob& job, bool counting, ph_render_stats& stats) {
     Impl& m = *impl_;
     stats = ph_render_stats{};
     const auto t0 = std::chrono::steady_clock::now();
-    const int pixels = job.width * job.height;
+    const int64_t pixels = int64_t(job.width) * job.height;
     if (pixels <= 0 || job.spp <= 0) return;
     if (m.serving) throw std::runtime_error("the engine is serving; a progressive render needs its own engine");
-    // Sub-streams per pixel: the largest divisor of spp not above the configured split.
-    int split = 1;
-    for (int k = 1; k <= std::min(m.cfg.sample_split, job.spp); k++)
-        if (job.spp % k == 0) split = k;
+    if (m.cfg.sample_split != 1 || m.cfg.path_slots != 0) {
+        // Sub-streams per pixel: the largest divisor of spp not above the configured split.
+        int split = 1;
+        for (int k = 1; k <= std::min(m.cfg.sample_split, job.spp); k++)
+            if (job.spp % k == 0) split = k;
+        // Paths in flight: one per pixel up to a cap of 4M slots (~900 MB of state), unless told.
+        const int64_t slots = m.cfg.path_slots > 0 ? m.cfg.path_slots : std::min<int64_t>(pixels, 1 << 22);
+        render_chunk(st, job, split, slots, m.cfg.graph_iterations, counting, stats);
+    } else {
+        const int64_t chunks = (job.spp + std::max<int64_t>(1, kChunkItems / pixels) - 1) / std::max<int64_t>(1, kChunkItems / pixels);
+        for (int64_t c = 0; c < chunks; c++) {
+            const int k0 = int(c * job.spp / chunks), k1 = int((c + 1) * job.spp / chunks);
+            WavefrontJob part = job;
+            part.frame0 = job.frame0 + uint32_t(k0);
+            part.spp = k1 - k0;
+            if (k0 > 0) part.albedo = part.nd = nullptr;  // the first sample's
+            if (!counting && m.cfg.finish_percent > 0 && pixels * part.spp <= kDirectItems)
+                render_direct(st, part, stats);
+            else
+                render_chunk(st, part, part.spp, kChunkSlots, std::min(kChunkGraph, m.cfg.graph_iterations), counting, stats);
+        }
+    }
+    stats.extend_launches = stats.iterations;
+    stats.shadow_launches = stats.iterations;
+    stats.shade_launches = stats.iterations * kClasses;
+    stats.samples = pixels * job.spp;
+    stats.ms_total = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
+}
+
+// A sample per lane (direct_kernel); adds to the statistics as finished paths.
+void WavefrontEngine::render_direct(hipStream_t st, const WavefrontJob& job, ph_render_stats& stats) {
+    Impl& m = *impl_;
+    const int pixels = job.width * job.height, items = pixels * job.spp;
+    const int* cls = job.mat_class;
+    WavefrontJob sub = job;
+    sub.split = job.spp;
+    if (sub.split > 1) {
+        m.part_sums.reserve(size_t(items));
+        sub.accum = m.part_sums.ptr;
+    }
+    m.direct_rays.allocate(2 * kDirectTallies);
+    hipLaunchKernelGGL(clear_tallies_kernel, dim3(1), dim3(2 * kDirectTallies), 0, st, m.direct_rays.ptr);
+    hipLaunchKernelGGL(job.scene.wide ? direct_kernel<true> : direct_kernel<false>, dim3((items + kDirectBlock - 1) / kDirectBlock), dim3(kDirectBlock), 0,
+                       st, m.params_of(sub, cls), m.direct_rays.ptr);
+    if (sub.split > 1)
+        hipLaunchKernelGGL(add_parts_kernel, dim3((pixels + kPartPixels - 1) / kPartPixels), dim3(kPartThreads), 0, st, m.part_sums.ptr, pixels, sub.split,
+                           job.accum);
+    PH_CHECK(hipGetLastError());
+    PH_CHECK(hipMemcpyAsync(m.host_direct, m.direct_rays.ptr, 2 * kDirectTallies * sizeof(unsigned long long), hipMemcpyDeviceToHost, st));
+    PH_CHECK(hipStreamSynchronize(st));
+    for (int k = 0; k < 2 * kDirectTallies; k++) stats.rays_finish += int64_t(m.host_direct[k]);
+    stats.finish_paths += items;
+}
+
+// One run of the bounce loop, `G` bounces at a time: the job's samples as `split` sub-streams per pixel (a divisor of
+// spp), at most `most` paths in flight.
+void WavefrontEngine::render_chunk(hipStream_t st, const WavefrontJob& job, int split, int64_t most, int G, bool counting, ph_render_stats& stats) {
+    Impl& m = *impl_;
+    const int pixels = job.width * job.height;
     const int64_t items = int64_t(pixels) * split;
     if (items > int64_t(INT32_MAX)) throw std::invalid_argument("pixels x sub-streams must stay below 2^31");
-    // Paths in flight: one per pixel up to a cap of 4M slots (~900 MB of state), never more than items.
-    const int slots = int(std::min<int64_t>(m.cfg.path_slots > 0 ? m.cfg.path_slots : std::min(pixels, 1 << 22), items));
+    const int slots = int(std::min(most, items));
     m.ensure_slots(slots);
     m.wide = job.scene.wide != nullptr;
     if (!job.mat_class) {
@@ -1337,7 +1453,7 @@ void WavefrontEngine::render(hipStream_t st, const WavefrontJob& job, bool count
     WavefrontJob sub = job;
     sub.split = split;
     if (split > 1) {
-        m.part_sums.allocate(size_t(items));
+        m.part_sums.reserve(size_t(items));
         sub.accum = m.part_sums.ptr;
     }
     const JobParams jp = m.params_of(sub, job.mat_class ? job.mat_class : m.mat_class.ptr);
@@ -1353,7 +1469,6 @@ void WavefrontEngine::render(hipStream_t st, const WavefrontJob& job, bool count
     m.compact<K_EXT, false>(st, m.state());
     PH_CHECK(hipGetLastError());
 
-    const int G = m.cfg.graph_iterations;
     // A sample takes at most max_depth bounces and a slot runs ceil(items / slots) items of spp/split samples.
     const int64_t bound = int64_t(job.spp / split) * int64_t(std::max(1, job.opt.max_depth)) * ((items + slots - 1) / slots) + 2 * G;
     double ms_extend = 0, ms_shadow = 0;
@@ -1375,24 +1490,19 @@ void WavefrontEngine::render(hipStream_t st, const WavefrontJob& job, bool count
     if (counting) PH_CHECK(hipMemcpy(tot, m.totals.ptr, sizeof(tot), hipMemcpyDeviceToHost));
     unsigned long long rays[5] = {0, 0, 0, 0, 0};
     PH_CHECK(hipMemcpy(rays, m.ray_totals.ptr, sizeof(rays), hipMemcpyDeviceToHost));
-    stats.rays_extend = int64_t(rays[0]);
-    stats.rays_shadow = int64_t(rays[1]) + m.host_counters[C_SHADOW];  // the last iteration's queue
-    stats.rays_finish = int64_t(rays[2] + rays[3]);
-    stats.finish_paths = int64_t(rays[4]);
-    stats.ms_extend = ms_extend;
-    stats.ms_shadow = ms_shadow;
-    stats.iterations = iterations;
-    stats.extend_launches = iterations;
-    stats.shadow_launches = iterations;
-    stats.shade_launches = iterations * kClasses;
-    stats.samples = int64_t(pixels) * job.spp;
-    stats.node_visits = int64_t(tot[0].nodes);
-    stats.tri_tests = int64_t(tot[0].tris);
-    stats.alpha_tests = int64_t(tot[0].alpha);
-    stats.shadow_node_visits = int64_t(tot[1].nodes);
-    stats.shadow_tri_tests = int64_t(tot[1].tris);
-    stats.shadow_alpha_tests = int64_t(tot[1].alpha);
-    stats.ms_total = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
+    stats.rays_extend += int64_t(rays[0]);
+    stats.rays_shadow += int64_t(rays[1]) + m.host_counters[C_SHADOW];  // the last iteration's queue
+    stats.rays_finish += int64_t(rays[2] + rays[3]);
+    stats.finish_paths += int64_t(rays[4]);
+    stats.ms_extend += ms_extend;
+    stats.ms_shadow += ms_shadow;
+    stats.iterations += iterations;
+    stats.node_visits += int64_t(tot[0].nodes);
+    stats.tri_tests += int64_t(tot[0].tris);
+    stats.alpha_tests += int64_t(tot[0].alpha);
+    stats.shadow_node_visits += int64_t(tot[1].nodes);
+    stats.shadow_tri_tests += int64_t(tot[1].tris);
+    stats.shadow_alpha_tests += int64_t(tot[1].alpha);
 }
 
 ph_wavefront_config WavefrontEngine::autotune(hipStream_t st, const WavefrontJob& job) {

@@ -157,3 +157,28 @@ def test_finishing_the_last_paths_one_per_thread_keeps_the_image(name, w, h, spp
         _, ref_acc, ref_g, _ = _render(scene, w, h, spp, gpu.ENGINE_MEGAKERNEL)
         assert on_acc.tobytes() == ref_acc.tobytes()
         assert on_g[0].tobytes() == ref_g[0].tobytes() and on_g[1].tobytes() == ref_g[1].tobytes()
+
+
+@pytest.mark.parametrize("name,w,h,spp,depth", [
+    ("cornell-c1", 1, 1, 1, 8), ("cornell-c1", 1, 1, 5, 8), ("materials", 17, 13, 3, 1), ("glass", 33, 65, 6, 8),
+    ("cornell-c1", 1024, 512, 2, 4), ("cornell-c1", 1025, 512, 2, 4), ("materials", 64, 48, 64, 8),
+    ("cornell-c1", 1920, 1080, 33, 3)])
+def test_default_launch_at_every_size_keeps_the_image(name, w, h, spp, depth):
+    """The default configuration renders in chunks of whole samples, small ones a sample per lane (up to 2^20
+    samples: 1024 x 512 x 2) and larger ones in bounces (several chunks past 2^26). The accumulation and the
+    G-buffer are the per-pixel kernel's bit for bit, on a second call too; so is an engine told its slots."""
+    scene = host.Scene.builtin(name).build()
+    rs = RenderSettings.make(w, h, max_depth=depth, rr_depth=3, seed=5)
+    cam = scene.camera_view(w / h)
+    planes = []
+    for engine, cfg, calls in ((gpu.ENGINE_MEGAKERNEL, {}, 2), (gpu.ENGINE_WAVEFRONT, {}, 2), (gpu.ENGINE_WAVEFRONT, dict(path_slots=7000), 2)):
+        r = uploaded(scene, w, h, engine=engine)
+        r.set_wavefront_config(**cfg)
+        for _ in range(calls):
+            r.render(cam, rs, spp)
+            assert r.stats().samples == w * h * spp
+        planes.append([gpu.copy_device_to_numpy(r.buffer_ptr(b), w * h * 16, np.float32, (h, w, 4)).tobytes()
+                       for b in (gpu.BUF_ACCUM, gpu.BUF_ALBEDO, gpu.BUF_NORMAL_DEPTH)])
+        r.close()
+    assert planes[0] == planes[1]
+    assert planes[0] == planes[2]
