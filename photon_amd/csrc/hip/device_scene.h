@@ -59,7 +59,7 @@ public:
         b += nodes_.bytes() + wide_.bytes() + tris_.bytes() + materials_.bytes() + indices_.bytes() + tri_emissive_.bytes();
         b += normals_.bytes() + uvs_.bytes() + tangents_.bytes() + srgb_lut_.bytes() + env_texels_.bytes();
         b += env_marginal_.bytes() + env_conditional_.bytes() + textures_.bytes() + texels_.bytes();
-        b += guide_marginal_.bytes() + guide_conditional_.bytes();
+        b += guide_marginal_.bytes() + guide_conditional_.bytes() + env_trig_.bytes();
         b += emissive_.bytes() + alias_.bytes() + punctual_.bytes();
         return b;
     }
@@ -143,7 +143,11 @@ public:
         // Guide tables for the sampling searches, one entry per power-of-two step of u.
         v.env_guide_marginal = v.env_guide_conditional = nullptr;
         v.env_guide_mh = v.env_guide_mw = 0;
+        v.env_trig = nullptr;
         if (env_n) {
+            env_trig_.allocate(size_t(d.env_height) + 4);
+            build_env_trig(st, d.env_rotation, d.env_height, env_trig_.ptr);
+            v.env_trig = env_trig_.ptr;
             auto pow2 = [](int n) {
                 int m = 1;
                 while (m < n && m < (1 << 16)) m <<= 1;
@@ -172,7 +176,7 @@ public:
 private:
     DevBuf<float4> nodes_, wide_, tris_, materials_;
     DevBuf<int> indices_, tri_emissive_;
-    DevBuf<float> normals_, uvs_, tangents_, srgb_lut_, env_texels_, env_marginal_, env_conditional_;
+    DevBuf<float> env_trig_, normals_, uvs_, tangents_, srgb_lut_, env_texels_, env_marginal_, env_conditional_;
     DevBuf<int> guide_marginal_, guide_conditional_;
     DevBuf<ph_texture_info> textures_;
     DevBuf<uint32_t> texels_;

@@ -6,8 +6,8 @@
 //     (src/core/math.h:52-124, src/core/sampling.h:9-99), built with -ffp-contract=off;
 //   * division and square root are IEEE correctly rounded (-fhip-fp32-correctly-rounded-divide-sqrt);
 //   * sin, cos, atan2, acos, exp and pow are evaluated in fp64 and rounded once to fp32, which gives
-//     the correctly rounded fp32 value except when the fp64 result lies within one fp64 ulp of an fp32
-//     rounding boundary (probability ~2^-29 per call). glibc's fp32 functions used by the CPU build are
+//     the correctly rounded fp32 value except when the fp64 result lies within an fp64 ulp or two of an
+//     fp32 rounding boundary (probability ~2^-27 per call). glibc's fp32 functions used by the CPU build are
 //     correctly rounded on all but a tiny fraction of inputs, so the two agree almost everywhere; fp64
 //     runs at half the fp32 rate on CDNA4, and these calls are a few per path vertex.
 #pragma once
@@ -18,6 +18,8 @@
 #include <type_traits>
 
 #define PH_DEV __device__ __forceinline__
+
+#include "dtrig.h"
 
 namespace phd {
 
@@ -61,16 +63,7 @@ constexpr float kInvTwoPi = 0.15915494309189533577f;
 constexpr float kInf = 1e30f;
 
 // ---- correctly rounded transcendentals -----------------------------------------------------------
-PH_DEV float sin_cr(float x) { return float(::sin(double(x))); }
-PH_DEV float cos_cr(float x) { return float(::cos(double(x))); }
-PH_DEV void sincos_cr(float x, float* s, float* c) {
-    double sd, cd;
-    ::sincos(double(x), &sd, &cd);
-    *s = float(sd);
-    *c = float(cd);
-}
-PH_DEV float atan2_cr(float y, float x) { return float(::atan2(double(y), double(x))); }
-PH_DEV float acos_cr(float x) { return float(::acos(double(x))); }
+// sincos_cr, atan2_cr and acos_cr: dtrig.h
 PH_DEV float exp_cr(float x) { return float(::exp(double(x))); }
 PH_DEV float pow_cr(float x, float y) { return float(::pow(double(x), double(y))); }
 

@@ -42,6 +42,9 @@ struct DScene {
     const int* env_guide_marginal;     // env_guide_mh + 1 entries
     const int* env_guide_conditional;  // env_h rows of env_guide_mw + 1 entries
     int env_guide_mh, env_guide_mw;
+    // Sine and cosine of minus the sky's rotation and of the rotation, then the sine of the polar angle at the
+    // middle of each row of the environment map (set whenever there is a map).
+    const float* env_trig;
     int num_tris, num_nodes, num_emissive, num_punctual;
     int top_nodes;  // nodes [0, top_nodes) are the top of the tree in breadth-first order
     int env_w, env_h;

@@ -242,9 +242,9 @@ PH_DEV int alias_pick(const ph_alias_entry* table, int n, float u, float* pmf) {
     return chosen;
 }
 
-PH_DEV f3 yaw(f3 d, float angle) {
-    float s, c;
-    sincos_cr(angle, &s, &c);
+// The sky's rotation: its sine and cosine are constants of the scene (DScene::env_trig).
+PH_DEV f3 yaw(const DScene& sc, f3 d, bool back) {
+    const float s = ldg(sc.env_trig + (back ? 0 : 2)), c = ldg(sc.env_trig + (back ? 1 : 3));
     return {c * d.x + s * d.z, d.y, -s * d.x + c * d.z};
 }
 
@@ -252,7 +252,7 @@ PH_DEV f3 env_texel(const DScene& s, int x, int y) { return n_at(s.env_texels, y
 
 PH_DEV f3 sky_radiance(const DScene& s, f3 dir) {
     if (!s.env_texels) return ld3(s.env_color) * s.env_intensity;
-    f2 uv = dir_to_latlong(yaw(dir, -s.env_rotation));
+    f2 uv = dir_to_latlong(yaw(s, dir, true));
     int x = int(uv.x * float(s.env_w));
     int y = int(uv.y * float(s.env_h));
     x = x < 0 ? 0 : (x >= s.env_w ? s.env_w - 1 : x);
@@ -290,14 +290,14 @@ PH_DEV int cdf_search_guided(const float* cdf, int n, const int* guide, int m, f
 
 PH_DEV float sky_pdf_dir(const DScene& s, f3 dir) {
     if (!s.env_texels) return 1.0f / (4.0f * kPi);
-    f3 d = yaw(dir, -s.env_rotation);
+    f3 d = yaw(s, dir, true);
     f2 uv = dir_to_latlong(d);
     float sin_theta = ssqrt(1 - d.y * d.y);
     if (sin_theta <= 0 || s.env_integral <= 0) return 0;
     int x = int(uv.x * float(s.env_w)), y = int(uv.y * float(s.env_h));
     x = x < 0 ? 0 : (x >= s.env_w ? s.env_w - 1 : x);
     y = y < 0 ? 0 : (y >= s.env_h ? s.env_h - 1 : y);
-    float row_sin = sin_cr((float(y) + 0.5f) / float(s.env_h) * kPi);
+    float row_sin = ldg(s.env_trig + 4 + y);
     float f = lum(env_texel(s, x, y)) * row_sin;
     float pdf_uv = f / s.env_integral;
     return pdf_uv / (2.0f * kPi * kPi * sin_theta);
@@ -321,10 +321,10 @@ PH_DEV bool sky_sample(const DScene& s, f2 u, f3& dir, float& pdf) {
     float du = r1 > r0 ? (u.x - r0) / (r1 - r0) : 0.5f;
     f2 uv = mk2((float(x) + du) / float(w), (float(y) + dv) / float(h));
     f3 d = latlong_to_dir(uv);
-    dir = yaw(d, s.env_rotation);
+    dir = yaw(s, d, false);
     float sin_theta = ssqrt(1 - d.y * d.y);
     if (sin_theta <= 1e-6f) return false;
-    float row_sin = sin_cr((float(y) + 0.5f) / float(h) * kPi);
+    float row_sin = ldg(s.env_trig + 4 + y);
     float f = lum(env_texel(s, x, y)) * row_sin;
     pdf = f / s.env_integral / (2.0f * kPi * kPi * sin_theta);
     return pdf > 0;

@@ -109,6 +109,8 @@ void mark_leaves(hipStream_t st, const float4* nodes, int num_nodes, int num_tri
 // Guide tables of `rows` CDFs of n + 1 entries each (row r at cdf + r * stride): guide[r * (m + 1) + k]
 // is the index the CDF search returns for u = k / m (m a power of two).
 void build_cdf_guides(hipStream_t st, const float* cdf, int rows, int n, size_t stride, int m, int* guide);
+// DScene::env_trig for a sky of `rows` rows.
+void build_env_trig(hipStream_t st, float rotation, int rows, float* out);
 
 // The same sample written as the compact G-buffer (photon_hip.h, ph_compact_gbuffer).
 void launch_sample_compact(hipStream_t st, const phd::DScene& s, const ph_camera_view& cam, int w, int h, uint32_t frame, uint32_t seed,

@@ -20,6 +20,19 @@ constexpr int kMegaDepth = 32;  // LDS stack entries per lane of the heat map
 //   * the 1080p render of that field runs at 479 Msamples/s instead of 329 (3 waves: 416).
 constexpr int kSampleWaves = 4;
 
+// The rotation is any angle, so these go through the library's fp64 functions.
+__global__ void env_trig_kernel(float rotation, int rows, float* out) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t < 2) {
+        const double angle = double(t == 0 ? -rotation : rotation);
+        out[2 * t] = float(::sin(angle));
+        out[2 * t + 1] = float(::cos(angle));
+    } else if (t < rows + 2) {
+        const int y = t - 2;
+        out[4 + y] = float(::sin(double((float(y) + 0.5f) / float(rows) * kPi)));
+    }
+}
+
 template <bool Wide>
 __global__ __launch_bounds__(kPixelBlock) __attribute__((amdgpu_waves_per_eu(kSampleWaves))) void render_kernel(DScene s, ph_camera_view cam, int w, int h, uint32_t frame0, int spp, uint32_t seed,
                                                              PathOpts opt, float4* accum, float4* albedo, float4* nd) {
@@ -292,6 +305,11 @@ void launch_sample(hipStream_t st, const DScene& s, const ph_camera_view& cam, i
 void build_cdf_guides(hipStream_t st, const float* cdf, int rows, int n, size_t stride, int m, int* guide) {
     const long long total = (long long)rows * (m + 1);
     hipLaunchKernelGGL(cdf_guide_kernel, dim3(unsigned((total + 255) / 256)), dim3(256), 0, st, cdf, rows, n, stride, m, guide);
+    PH_CHECK(hipGetLastError());
+}
+
+void build_env_trig(hipStream_t st, float rotation, int rows, float* out) {
+    hipLaunchKernelGGL(env_trig_kernel, dim3((rows + 2 + 255) / 256), dim3(256), 0, st, rotation, rows, out);
     PH_CHECK(hipGetLastError());
 }
 

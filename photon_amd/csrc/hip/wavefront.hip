@@ -636,7 +636,7 @@ __global__ __launch_bounds__(256) void miss_kernel(Work work, State st, int* cou
 
 // One path vertex (integrator.h:178-260) for the slots of one material class.
 template <int Lobes, bool Multi>
-__global__ __launch_bounds__(256) void shade_kernel(Work work, State st, int* counters, int cls, int bins) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void shade_kernel(Work work, State st, int* counters, int cls, int bins) {
     const int n = counters[C_CLASS + cls];
     const int* queue = st.q_class[cls];
     const JobParams single = single_job<Multi>(work);
@@ -1218,9 +1218,9 @@ struct WavefrontEngine::Impl {
         const auto blocks_for = [&](int most, int block) { return std::max(1, std::min(most, (slots + block - 1) / block)); };
         const bool over_wide = wide && !count && (Multi || cfg.lds_nodes == 0);
         const int tgrid = blocks_for(cus * std::max(1, cfg.blocks_per_cu) * (over_wide ? 4 : 1), cfg.block);
-        // Shading: 4 blocks of 256 threads per CU. The shading kernels use 232 VGPRs (2 waves per SIMD), so
-        // half of the blocks start as the others finish their share. Compiling them for 6 or 8 waves (with a
-        // grid to match) spills and was slower: 940 and 897 against 995 Msamples/s.
+        // Shading: 4 blocks of 256 threads per CU, all of them resident: the shading kernels need 140 VGPRs since the
+        // bounded trigonometry (dtrig.h; 232 before, 2 waves per SIMD), and 128 spill at most 8. 1080p, 64 samples, 1M
+        // triangles: 79.6 ms at 3 waves per SIMD, 75.0 at 4, 78.4 at 5; 8 to 32 blocks per CU 74.4 to 75.0.
         const int sgrid = blocks_for(cus * 4, 256);
         const State s = state();
         const Work w = work();
