@@ -58,6 +58,25 @@ struct Job {
 
 }  // namespace
 
+// A finished job's image: each pixel's partial sums in sub-stream order (one: the accumulation itself), over the
+// samples. On the device: the host's sum of 16-byte partial sums read them all over the bus and was most of a
+// result's time.
+__global__ __launch_bounds__(256) void resolve_kernel(const float4* sums, int pixels, int split, float inv, float* rgb) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i >= pixels) return;
+    const float4* part = sums + size_t(i) * size_t(split);
+    float r = part->x, g = part->y, b = part->z;
+    for (int p = 1; p < split; p++) {
+        const float4 v = part[p];
+        r += v.x;
+        g += v.y;
+        b += v.z;
+    }
+    rgb[3 * size_t(i)] = r * inv;
+    rgb[3 * size_t(i) + 1] = g * inv;
+    rgb[3 * size_t(i) + 2] = b * inv;
+}
+
 // One engine with its own stream and slots. The main lane runs every job by default; the express lane
 // (when configured) runs the jobs of at most `express_samples` samples on a small slot pool of its own,
 // concurrently with the main lane, so that a short job's bounces are not each as long as an iteration
@@ -80,6 +99,7 @@ struct ph_server {
     Lane lanes[2];  // 0: main, 1: express
     std::vector<std::unique_ptr<ServedScene>> scenes;
     std::vector<std::unique_ptr<Job>> jobs;
+    DevBuf<float> image;  // the result being read: as large as the largest read so far
     int64_t mem_used = 0;
     int finished = 0;
     std::chrono::steady_clock::time_point t0 = std::chrono::steady_clock::now();
@@ -377,24 +397,12 @@ int ph_server_result(ph_server* s, int job, float* rgb) {
     if (j.status.state != PH_JOB_DONE) return set_error(j.status.state == PH_JOB_RELEASED ? "the job's result was already read" : "the job is not done");
     return guarded([&] {
         const size_t n = size_t(j.status.pixels);
-        std::vector<float4> raw(size_t(j.items));
-        PH_CHECK(hipMemcpyAsync(raw.data(), j.accum.ptr, raw.size() * sizeof(float4), hipMemcpyDeviceToHost, s->stream()));
+        s->image.reserve(3 * n);
+        hipLaunchKernelGGL(resolve_kernel, dim3(unsigned((n + 255) / 256)), dim3(256), 0, s->stream(), j.accum.ptr, j.status.pixels, j.split,
+                           1.0f / float(j.desc.spp), s->image.ptr);
+        PH_CHECK(hipGetLastError());
+        PH_CHECK(hipMemcpyAsync(rgb, s->image.ptr, 3 * n * sizeof(float), hipMemcpyDeviceToHost, s->stream()));
         PH_CHECK(hipStreamSynchronize(s->stream()));
-        const float inv = 1.0f / float(j.desc.spp);
-        for (size_t i = 0; i < n; i++) {
-            // The pixel's partial sums in sub-stream order (one: the accumulation itself).
-            const float4* part = raw.data() + i * size_t(j.split);
-            float r = part->x, g = part->y, b = part->z;
-            for (int p = 1; p < j.split; p++) {
-                const float4& v = part[p];
-                r += v.x;
-                g += v.y;
-                b += v.z;
-            }
-            rgb[3 * i] = r * inv;
-            rgb[3 * i + 1] = g * inv;
-            rgb[3 * i + 2] = b * inv;
-        }
         j.accum.release();
         s->mem_used -= int64_t(j.bytes);
         j.status.state = PH_JOB_RELEASED;
