@@ -13,8 +13,8 @@
 //     (cost, candidate) pairs to the same first minimum.
 //   * the partition is std::partition's: the k-th element on the wrong side counted from the front
 //     swaps with the k-th counted from the back; ranks come from scans, so it runs in parallel.
-// Large nodes (more than kSubtree triangles) are split level by level by multi-block passes with the
-// per-node decisions on the host; every subtree of at most kSubtree triangles is then built level by
+// Large nodes (more than subtree_bound triangles) are split level by level by multi-block passes with the
+// per-node decisions on the host; every subtree of at most subtree_bound triangles is then built level by
 // level by one block, a wave per node. The node indices of the build tree differ from the host's, but
 // the flattening, also on the device, numbers nodes by tree structure only.
 #include <algorithm>
@@ -34,8 +34,18 @@ namespace {
 constexpr float kBoxInf = 1e30f;  // the host builder's empty box bound
 constexpr int kMaxBins = 64;
 constexpr int kChunk = 2048;    // triangles per block of the large-node passes
-constexpr int kSubtree = 2048;  // subtrees of at most this many triangles are built by one block each
+constexpr int kSubtree = 2048, kSubtreeMin = 256;  // range of subtree_bound
 static_assert(kSubtree <= kChunk, "the subtree kernel's level lists hold kChunk entries");
+
+// Subtrees of at most this many triangles are built by one block each. A block's time grows with its subtree, and a
+// split of the large nodes costs the host a round trip a level, so the bound follows the build: about 200 blocks on the
+// 256 CUs. Measured with 256 / 512 / 1024 / 2048, ms: 4,096 triangles 1.22 / 1.45 / 2.04 / 3.43; 32,768 2.33 / 2.47 /
+// 3.05 / 4.35; 65,536 3.99 / 3.85 / 4.33 / 5.73; 131,072 6.27 / 5.64 / 5.51 / 6.73; 256,000 9.34 / 9.15 / 8.76 / 8.74.
+int subtree_bound(int n) {
+    int bound = kSubtreeMin;
+    while (bound < kSubtree && 2 * bound * 128 <= n) bound *= 2;
+    return bound;
+}
 constexpr int kThreads = 256;
 
 // The host's std::fmin / std::fmax for finite values: the second operand unless the first is strictly
@@ -735,7 +745,8 @@ int64_t bvh_build_device(const float* positions, int num_vertices, const int* in
     std::vector<Big> level{{0, 0, n, 0}};
     std::vector<Pending> small;
     int next_node = 1;
-    if (n <= kSubtree) {
+    const int bound = subtree_bound(n);
+    if (n <= bound) {
         small.push_back(Pending{0, 0, n, 0});
         level.clear();
     }
@@ -868,7 +879,7 @@ int64_t bvh_build_device(const float* positions, int num_vertices, const int* in
                 for (int side = 0; side < 2; side++) {
                     const int cf = side == 0 ? first : m, cc = side == 0 ? m - first : first + count - m;
                     const int idx = side == 0 ? rec.left : rec.right;
-                    if (cc > kSubtree)
+                    if (cc > bound)
                         next.push_back(Big{idx, cf, cc, nd.depth + 1});
                     else
                         small.push_back(Pending{idx, cf, cc, nd.depth + 1});
