@@ -126,3 +126,16 @@ def test_wavefront_image_over_either_walk(w, h, spp, split):
         r.update_lights(scene)
     assert images[0].tobytes() == images[1].tobytes() == images[2].tobytes()
     r.close()
+
+
+@pytest.mark.parametrize("n", [1, 129, 786431, 786432, 1000003])
+def test_any_hit_launches_report_the_same_hits(n):
+    """Few any-hit rays run in blocks, many (from 786,432 on) in a grid with refilled lanes: both report the counting
+    walk's hits."""
+    scene = host.Scene.spheres(12, box=12.0, alpha_fraction=0.3, seed=4).build()
+    r = uploaded(scene)
+    rays = scene.shadow_rays(n, seed=3)
+    got = trace_on_gpu(r, rays, anyhit=True)
+    want, _ = trace_on_gpu(r, rays, anyhit=True, counts=True)
+    assert got.tobytes() == want.tobytes()
+    r.close()
