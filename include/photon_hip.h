@@ -235,7 +235,7 @@ int ph_svgf_run_compact(ph_svgf* f, const ph_compact_gbuffer* in, const ph_camer
  * the same nine passes as ph_svgf_run on one frame of at most PH_SVGF_STATIC_MAX_PIXELS pixels (larger
  * frames fail with a message). The frame-local planes (illumination, moments, two a-trous planes: 64
  * bytes per pixel) live in one static device array that each GPU the library runs on holds until the
- * process ends (PH_SVGF_STATIC_MAX_PIXELS * 64 bytes = 92 MB). The history that ph_svgf keeps inside
+ * process ends (PH_SVGF_STATIC_MAX_PIXELS * 70 bytes = 101 MB). The history that ph_svgf keeps inside
  * the object is the caller's instead: `history_dev` holds four float4 planes of width*height pixels
  * (illumination + history length, moments, normal+depth, position+material), is read when
  * `has_history` is nonzero (0 for the first frame, as after ph_svgf_reset) and is rewritten by the call.

@@ -62,12 +62,15 @@ PH_DEV bool reproject(const ph_camera_view& c, f3 p, int w, int h, float& px, fl
 // normal+depth and position+material planes.
 struct RefIn {
     const float4 *color, *albedo, *nd, *pos, *emission;
+    float* materials;  // pos[].w packed, from the temporal pass on: the later passes need no other part of the position
     PH_DEV f3 color3(int i) const { return xyz(color[i]); }
     PH_DEV f3 albedo3(int i) const { return xyz(albedo[i]); }
     PH_DEV f3 emission3(int i) const { return xyz(emission[i]); }
     PH_DEV float4 ndz(int i) const { return nd[i]; }
     PH_DEV float4 ndz_w(int i) const { return nd[i]; }
-    PH_DEV float mat(int i) const { return pos[i].w; }
+    PH_DEV float first_mat(int i) const { return pos[i].w; }
+    PH_DEV void pack_mat(int i, float m) const { materials[i] = m; }
+    PH_DEV float mat(int i) const { return materials[i]; }
     PH_DEV f3 position(int i, int, int) const { return xyz(pos[i]); }
     PH_DEV float4 raw_color(int i) const { return color[i]; }
 };
@@ -103,6 +106,8 @@ struct CompactIn {
         const f3 n = oct_decode_approx(normal[i]);
         return make_float4(n.x, n.y, n.z, depth[i]);
     }
+    PH_DEV float first_mat(int i) const { return mat(i); }
+    PH_DEV void pack_mat(int, float) const {}
     PH_DEV float mat(int i) const { return float(material[i]); }
     PH_DEV f3 position(int i, int x, int y) const { return centre_position(cam, x, y, w, h, depth[i]); }
     PH_DEV float4 raw_color(int i) const {
@@ -138,11 +143,15 @@ constexpr int kRowX = 64, kRowY = 4;
 template <class In, class Hist>
 __global__ __launch_bounds__(kRowX* kRowY) void temporal_kernel(In in, ph_camera_view prev_cam, int w, int h, int has_history, float alpha_c,
                                                            float alpha_m, const float4* prev_illum, const float4* prev_moments, Hist prev,
-                                                           float4* out_illum, float4* out_moments) {
+                                                           float4* out_illum, float4* out_moments, float4* out_filter, int* short_history) {
     const int x = blockIdx.x * kRowX + threadIdx.x, y = blockIdx.y * kRowY + threadIdx.y;
+    const int block = blockIdx.y * gridDim.x + blockIdx.x;
+    if (threadIdx.x + threadIdx.y == 0) short_history[block] = 0;
+    __syncthreads();
     if (x >= w || y >= h) return;
     const int i = y * w + x;
-    const float mat = in.mat(i);
+    const float mat = in.first_mat(i);
+    in.pack_mat(i, mat);
     const f3 cur = demod(in.color3(i), in.emission3(i), in.albedo3(i));
     const float l = lum(cur);
     f3 hist_c = mk3(0);
@@ -198,6 +207,8 @@ __global__ __launch_bounds__(kRowX* kRowY) void temporal_kernel(In in, ph_camera
     const float variance = fmaxf(0.0f, m1 - m0 * m0);
     out_illum[i] = make_float4(c.x, c.y, c.z, len);
     out_moments[i] = make_float4(m0, m1, variance, 0.0f);
+    out_filter[i] = make_float4(c.x, c.y, c.z, variance);
+    if (len < 4.0f && mat >= 0) short_history[block] = 1;
 }
 
 // The 7x7 estimate of one short-history pixel (svgf.cu:96-132): moments and illumination of the taps
@@ -240,27 +251,33 @@ PH_DEV float4 spatial_estimate(int x, int y, int w, int h, float mat, float4 ndc
     return make_float4(c.x, c.y, c.z, var);
 }
 
-// Variance pass. Pixels whose history has reached 4 frames keep their temporal estimate; the others take
-// the 7x7 spatial estimate. A block with no such pixel (the common case once the camera has settled)
-// only copies; any other stages the 22x22 halo of normal+depth and material in LDS once (gathering the
-// taps of a block's few short-history pixels through the caches instead measured slower).
+// Variance pass. Pixels whose history has reached 4 frames keep their temporal estimate, which the temporal pass has
+// written; the others take the 7x7 spatial estimate. A block of the temporal pass with none of these (the common case
+// once the camera has settled) is known by its flag; any other tile stages the 22x22 halo of normal+depth and
+// material in LDS once (gathering the taps of a block's few short-history pixels through the caches instead
+// measured slower).
 
 template <class In>
 __global__ __launch_bounds__(TX* TY) void variance_kernel(In in, int w, int h, const float4* illum, const float4* moments, float phi_normal,
-                                                           float4* out) {
+                                                           const int* short_history, float4* out) {
     constexpr int R = 3, SX = TX + 2 * R, SY = TY + 2 * R;
+    static_assert(kRowX % TX == 0 && TY % kRowY == 0, "a tile lies in one column of the temporal pass's blocks");
     __shared__ float4 s_nd[SY][SX];
     __shared__ float s_mat[SY][SX];
+    const int row_blocks = (w + kRowX - 1) / kRowX, last = (h + kRowY - 1) / kRowY;
+    int any = 0;
+    for (int k = 0; k < TY / kRowY; k++) {
+        const int by = int(blockIdx.y) * (TY / kRowY) + k;
+        if (by < last) any |= short_history[by * row_blocks + int(blockIdx.x) * TX / kRowX];
+    }
+    if (!any) return;
     const int x = blockIdx.x * TX + threadIdx.x, y = blockIdx.y * TY + threadIdx.y;
     const bool inside = x < w && y < h;
     const int i = inside ? y * w + x : 0;
     const float4 c = inside ? illum[i] : make_float4(0, 0, 0, 4.0f);
     const float mat = inside ? in.mat(i) : -1.0f;
     const bool spatial = inside && c.w < 4.0f && mat >= 0;
-    if (!__syncthreads_or(spatial)) {
-        if (inside) out[i] = make_float4(c.x, c.y, c.z, moments[i].z);
-        return;
-    }
+    if (!__syncthreads_or(spatial)) return;
     const int bx = blockIdx.x * TX - R, by = blockIdx.y * TY - R;
     for (int t = threadIdx.y * TX + threadIdx.x; t < SX * SY; t += TX * TY) {
         const int sy = t / SX, sx = t % SX;
@@ -272,14 +289,11 @@ __global__ __launch_bounds__(TX* TY) void variance_kernel(In in, int w, int h, c
         }
     }
     __syncthreads();
-    if (!inside) return;
+    if (!spatial) return;
     const int ly = threadIdx.y + R, lx = threadIdx.x + R;
-    float4 r = make_float4(c.x, c.y, c.z, moments[i].z);
-    if (spatial)
-        r = spatial_estimate(
-            x, y, w, h, mat, s_nd[ly][lx], [&](int dx, int dy) { return s_nd[ly + dy][lx + dx]; }, [&](int dx, int dy) { return s_mat[ly + dy][lx + dx]; },
-            illum, moments, phi_normal, c, r.w);
-    out[i] = r;
+    out[i] = spatial_estimate(
+        x, y, w, h, mat, s_nd[ly][lx], [&](int dx, int dy) { return s_nd[ly + dy][lx + dx]; }, [&](int dx, int dy) { return s_mat[ly + dy][lx + dx]; },
+        illum, moments, phi_normal, c, moments[i].z);
 }
 
 // What a pass does with its result besides writing its output plane: the history of the next frame is
@@ -473,7 +487,11 @@ struct PassPlanes {
     bool has_history;
     float4 *prev_illum, *prev_moments;
     float4 *illum, *moments, *filter0, *filter1;
+    int* short_history;  // per block of the temporal pass
 };
+
+// Blocks of the temporal pass.
+dim3 row_grid(int w, int h) { return dim3((w + kRowX - 1) / kRowX, (h + kRowY - 1) / kRowY); }
 
 // Grid of atrous_lattice_kernel: 64-pixel column groups by (groups of kLatticeRows lattice rows) x residues.
 dim3 lattice_grid(int w, int h, int step) {
@@ -490,9 +508,9 @@ void run_passes(const PassPlanes& pl, hipStream_t st, const In& in, const Hist& 
     float4 *illum = pl.illum, *moments = pl.moments, *filter[2] = {pl.filter0, pl.filter1};
     const dim3 tile(TX, TY), grid((w + TX - 1) / TX, (h + TY - 1) / TY);
     const int lin = 256, lgrid = (n + lin - 1) / lin;
-    hipLaunchKernelGGL((temporal_kernel<In, Hist>), dim3((w + kRowX - 1) / kRowX, (h + kRowY - 1) / kRowY), dim3(kRowX, kRowY), 0, st, in, prev_cam, w, h, int(pl.has_history), s.alpha_color, s.alpha_moments,
-                       prev_illum, prev_moments, prev, illum, moments);
-    hipLaunchKernelGGL((variance_kernel<In>), grid, tile, 0, st, in, w, h, illum, moments, s.phi_normal, filter[0]);
+    hipLaunchKernelGGL((temporal_kernel<In, Hist>), row_grid(w, h), dim3(kRowX, kRowY), 0, st, in, prev_cam, w, h, int(pl.has_history), s.alpha_color,
+                       s.alpha_moments, prev_illum, prev_moments, prev, illum, moments, filter[0], pl.short_history);
+    hipLaunchKernelGGL((variance_kernel<In>), grid, tile, 0, st, in, w, h, illum, moments, s.phi_normal, pl.short_history, filter[0]);
     int src = 0;
     const int iters = s.atrous_iterations;
     for (int it = 0; it < iters; it++) {
@@ -529,14 +547,18 @@ void run_passes(const PassPlanes& pl, hipStream_t st, const In& in, const Hist& 
 }
 
 PassPlanes planes_of(const SvgfState& f) {
-    return PassPlanes{f.w, f.h, f.has_history, f.plane[0].ptr, f.plane[1].ptr, f.plane[4].ptr, f.plane[5].ptr, f.plane[6].ptr, f.plane[7].ptr};
+    return PassPlanes{f.w, f.h, f.has_history, f.plane[0].ptr, f.plane[1].ptr, f.plane[4].ptr, f.plane[5].ptr, f.plane[6].ptr, f.plane[7].ptr,
+                      f.short_history.ptr};
 }
 
 // Frame-local planes of the allocation-free entry point: illumination, moments and the two a-trous
 // planes of up to kStaticSvgfPixels pixels, in one file-scope device array that every GPU holds from
 // the library's load until the process ends. Host code never names the array: it uses the address
 // that hipGetSymbolAddress returns on each device.
-__device__ __align__(256) float4 scratch[4 * size_t(PH_SVGF_STATIC_MAX_PIXELS)];
+// Behind the planes lie the packed materials (a float each) and the temporal pass's flags: of a w x h frame
+// (w/64 + 1)(h/4 + 1) at most, which is below half an int a pixel plus 4.
+constexpr size_t kStaticPixels = size_t(PH_SVGF_STATIC_MAX_PIXELS);
+__device__ __align__(256) float4 scratch[4 * kStaticPixels + kStaticPixels / 4 + kStaticPixels / 8 + 4];
 
 constexpr int kMaxDevices = 64;
 float4* g_scratch[kMaxDevices] = {};
@@ -569,6 +591,8 @@ void svgf_resize(SvgfState& f, int width, int height) {
         p.allocate(n);
         PH_CHECK(hipMemset(p.ptr, 0, n * sizeof(float4)));
     }
+    f.materials.allocate(n);
+    f.short_history.allocate(size_t(row_grid(width, height).x) * row_grid(width, height).y);
     f.has_history = false;
 }
 
@@ -578,7 +602,7 @@ void svgf_run(SvgfState& f, hipStream_t st, const ph_svgf_input& input, const ph
     f.history_compact = false;
     const RefIn in{reinterpret_cast<const float4*>(input.color_dev), reinterpret_cast<const float4*>(input.albedo_dev),
                    reinterpret_cast<const float4*>(input.normal_depth_dev), reinterpret_cast<const float4*>(input.position_dev),
-                   reinterpret_cast<const float4*>(input.emission_dev)};
+                   reinterpret_cast<const float4*>(input.emission_dev), f.materials.ptr};
     run_passes(planes_of(f), st, in, RefHist{f.plane[2].ptr, f.plane[3].ptr}, prev_cam, s, output);
     f.has_history = true;
 }
@@ -590,10 +614,12 @@ void svgf_run_static(hipStream_t st, int width, int height, const ph_svgf_input&
     if (n > size_t(PH_SVGF_STATIC_MAX_PIXELS)) throw std::runtime_error("frame larger than the static SVGF scratch");
     float4* base = static_scratch();
     // History: the caller's four planes (illumination + length, moments, normal+depth, position+material).
-    const PassPlanes pl{width, height, has_history, history, history + n, base, base + n, base + 2 * n, base + 3 * n};
+    float* materials = reinterpret_cast<float*>(base + 4 * n);
+    const PassPlanes pl{width,    height,       has_history,  history, history + n, base, base + n, base + 2 * n, base + 3 * n,
+                        reinterpret_cast<int*>(materials + n)};
     const RefIn in{reinterpret_cast<const float4*>(input.color_dev), reinterpret_cast<const float4*>(input.albedo_dev),
                    reinterpret_cast<const float4*>(input.normal_depth_dev), reinterpret_cast<const float4*>(input.position_dev),
-                   reinterpret_cast<const float4*>(input.emission_dev)};
+                   reinterpret_cast<const float4*>(input.emission_dev), materials};
     run_passes(pl, st, in, RefHist{history + 2 * n, history + 3 * n}, prev_cam, s, output);
 }
 

@@ -15,6 +15,8 @@ struct SvgfState {
     // The previous frame's geometry when the input is the compact G-buffer (planes 2 and 3 hold it for
     // the float4 input); `history_compact` says which format the stored frame is in.
     bool history_compact = false;
+    DevBuf<float> materials;    // this frame's, packed from a float4 position plane
+    DevBuf<int> short_history;  // per block of the temporal pass: whether a pixel's history is short
     DevBuf<float> prev_depth;
     DevBuf<uint32_t> prev_normal;
     DevBuf<int> prev_material;
