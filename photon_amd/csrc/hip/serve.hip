@@ -59,8 +59,8 @@ struct Job {
 }  // namespace
 
 // A finished job's image: each pixel's partial sums in sub-stream order (one: the accumulation itself), over the
-// samples. On the device: the host's sum of 16-byte partial sums read them all over the bus and was most of a
-// result's time.
+// samples. On the device: the host's sum read all 16-byte partial sums over the bus, into fresh pages (eight jobs of
+// 65K to 921K pixels: 25 ms, 5 ms with this kernel and the 12-byte pixels copied).
 __global__ __launch_bounds__(256) void resolve_kernel(const float4* sums, int pixels, int split, float inv, float* rgb) {
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= pixels) return;

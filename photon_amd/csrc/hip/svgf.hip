@@ -255,7 +255,8 @@ PH_DEV float4 spatial_estimate(int x, int y, int w, int h, float mat, float4 ndc
 // written; the others take the 7x7 spatial estimate. A block of the temporal pass with none of these (the common case
 // once the camera has settled) is known by its flag; any other tile stages the 22x22 halo of normal+depth and
 // material in LDS once (gathering the taps of a block's few short-history pixels through the caches instead
-// measured slower).
+// measured slower). Bound by memory: copying the plane here and reading materials from the position plane, a
+// 1600x900 float4 frame took 0.370 ms; with the temporal pass writing both it takes 0.351.
 
 template <class In>
 __global__ __launch_bounds__(TX* TY) void variance_kernel(In in, int w, int h, const float4* illum, const float4* moments, float phi_normal,
