@@ -572,7 +572,7 @@ int ph_trace(ph_renderer* r, const ph_ray* rays, int n, int anyhit, ph_hit* hits
     if (!r->uploaded) return fail("no scene uploaded");
     return guarded([&] {
         ph_renderer& m = *r;
-        // Closest hits do not depend on the walk, so they go over the wide nodes. Any-hit results are the first hit of
+        // Closest hits do not depend on the walk (dwide.h names the exception), so they go over the wide nodes. Any-hit results are the first hit of
         // the binary walk's order, and counts are its counts. Any-hit rays end at very different times: with more than
         // one and a half rays for each of the chip's 524,288 lanes a fixed grid with refilled lanes is faster
         // (1,000,003 rays into 16K / 64K / 256K triangles 0.33 / 0.48 / 0.50 ms in blocks, 0.31 / 0.43 / 0.49 refilled;

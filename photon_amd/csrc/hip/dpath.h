@@ -46,7 +46,7 @@ template <int Block, bool Wide>
 using PathStack = StackShape<Block, Wide ? 20 : 32, Wide>;
 
 // A path's closest-hit and any-hit queries, over the wide nodes or (a scene outside their limits, or a
-// counting kernel) the binary ones: the answers are the same.
+// counting kernel) the binary ones: the answers are the same, but for the rays that dwide.h names.
 template <bool AnyHit, bool Count, int Depth, int Block>
 PH_DEV bool path_query(const DScene& s, f3 o, f3 d, float tmax, HitRec& hit, WideStack<Depth, Block>& stack, TraceCount*) {
     return traverse_wide<AnyHit, !AnyHit>(trace_scene(s), o, d, tmax, hit, stack);

@@ -19,12 +19,15 @@
 // The runtime calls are the subset the build code uses; copies and fills are synchronous.
 #pragma once
 
+#if defined(__SANITIZE_ADDRESS__)
 #include <sanitizer/asan_interface.h>
 #include <sanitizer/common_interface_defs.h>
+#endif
 #include <sys/mman.h>
 
 #include <algorithm>
 #include <atomic>
+#include <cmath>
 #include <cstdint>
 #include <cstdio>
 #include <cstdlib>
@@ -54,13 +57,19 @@ struct dim3 {
 struct float2 {
     float x, y;
 };
-struct float4 {
+struct alignas(16) float4 {
     float x, y, z, w;
+};
+struct alignas(16) int4 {
+    int x, y, z, w;
 };
 inline float2 make_float2(float x, float y) { return float2{x, y}; }
 inline float4 make_float4(float x, float y, float z, float w) { return float4{x, y, z, w}; }
+inline int4 make_int4(int x, int y, int z, int w) { return int4{x, y, z, w}; }
 inline int __float_as_int(float f) { return __builtin_bit_cast(int, f); }
 inline float __int_as_float(int i) { return __builtin_bit_cast(float, i); }
+inline unsigned __float_as_uint(float f) { return __builtin_bit_cast(unsigned, f); }
+inline float __uint_as_float(unsigned i) { return __builtin_bit_cast(float, i); }
 inline int __popcll(unsigned long long x) { return __builtin_popcountll(x); }
 inline int min(int a, int b) { return a < b ? a : b; }
 inline int max(int a, int b) { return a > b ? a : b; }
@@ -352,6 +361,7 @@ void launch_kernel(dim3 grid, dim3 block, F kernel, A... args) {
 #define blockIdx (::hipcpu::tl_block_idx)
 #define blockDim (::hipcpu::tl_block_dim)
 #define gridDim (::hipcpu::tl_grid_dim)
+#define __lane_id() int(threadIdx.x & 63)
 #define __syncthreads() ::hipcpu::block_barrier()
 #define __builtin_amdgcn_wave_barrier() ::hipcpu::wave_barrier()
 #define hipLaunchKernelGGL(K, G, B, S, ST, ...) ::hipcpu::launch_kernel(dim3(G), dim3(B), K, __VA_ARGS__)
@@ -375,6 +385,7 @@ T __shfl_xor(T v, int m) {
 inline unsigned long long __ballot(bool p) { return ::hipcpu::ballot(p); }
 
 inline int atomicAdd(int* p, int v) { return __atomic_fetch_add(p, v, __ATOMIC_SEQ_CST); }
+inline int atomicOr(int* p, int v) { return __atomic_fetch_or(p, v, __ATOMIC_SEQ_CST); }
 inline int atomicMin(int* p, int v) {
     int old = __atomic_load_n(p, __ATOMIC_SEQ_CST);
     while (v < old && !__atomic_compare_exchange_n(p, &old, v, false, __ATOMIC_SEQ_CST, __ATOMIC_SEQ_CST)) {
