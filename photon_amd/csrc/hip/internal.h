@@ -101,7 +101,7 @@ int64_t bvh_build_device(const float* positions, int num_vertices, const int* in
 
 // ---- wide_build.hip -----------------------------------------------------------------------------------
 // The scene's four-wide nodes (dwide.h) from its binary nodes. False, with `wide` empty, where the format's limits
-// (leaf size, triangle count, coordinates) are exceeded: such a scene is traced over the binary nodes.
+// (leaf size, triangle count, coordinates, boxes that nest) are exceeded: such a scene is traced over the binary nodes.
 bool build_wide_nodes(hipStream_t st, const float4* nodes, int num_nodes, int num_tris, DevBuf<float4>& wide);
 // Writes each triangle's leaf into the triangle's unused word.
 void mark_leaves(hipStream_t st, const float4* nodes, int num_nodes, int num_tris, float4* tris);

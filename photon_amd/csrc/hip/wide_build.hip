@@ -54,14 +54,26 @@ PH_DEV int collapse(const float4* nodes, int num_nodes, int i, Child* c) {
     return n;
 }
 
+PH_DEV bool inside(const Child& c, const Child& box) {
+    return c.lo.x >= box.lo.x && c.lo.y >= box.lo.y && c.lo.z >= box.lo.z && c.hi.x <= box.hi.x && c.hi.y <= box.hi.y && c.hi.z <= box.hi.z;
+}
+
 // Every binary node's interior children in its wide node (-1: none), and whether all of them and its leaves lie
-// within the format's limits (status[1] becomes nonzero where not).
+// within the format's limits (status[1] becomes nonzero where not). The binary nodes' boxes must nest: a wide node
+// leaves out the boxes between its node and the descendants it holds, which the binary walk tests.
 __global__ __launch_bounds__(256) void wide_children_kernel(const float4* nodes, int num_nodes, int num_tris, int4* children, int* status) {
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= num_nodes) return;
     Child c[4];
-    const int n = collapse(nodes, num_nodes, i, c);
     bool ok = true;
+    const int sides = add_children(nodes, i, c, 0);
+    for (int k = 0; k < sides; k++) {
+        if (!interior(c[k]) || c[k].link >= num_nodes) continue;
+        Child below[2];
+        const int m = add_children(nodes, c[k].link, below, 0);
+        for (int j = 0; j < m; j++) ok = ok && inside(below[j], c[k]);
+    }
+    const int n = collapse(nodes, num_nodes, i, c);
     int inner[4] = {-1, -1, -1, -1}, m = 0;
     for (int k = 0; k < n; k++) {
         const f3 a = c[k].lo, b = c[k].hi;

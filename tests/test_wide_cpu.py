@@ -86,3 +86,40 @@ def test_hits_along_triangles_planes_differ_only_where_the_distance_is_lost(lib,
         assert np.all(got["t"][at] > want["t"][at])
         _, want, got, _ = hipcpu_wide.walk(lib, nodes, tris, rays, anyhit=True)
         assert np.array_equal(want["tri"] >= 0, got["tri"] >= 0)
+
+
+def _rays_through(rng, n):
+    r = np.zeros(n, RAY_DTYPE)
+    d = rng.normal(size=(n, 3))
+    r["d"] = d / np.linalg.norm(d, axis=1, keepdims=True)
+    r["o"] = rng.uniform(-1, 1, (n, 3)) - 4 * r["d"]
+    r["tmax"] = 1e30
+    return r
+
+
+def test_scenes_of_this_librarys_builders_have_wide_nodes(lib):
+    for scene in (host.Scene.builtin("cornell-c1"), host.Scene.builtin("materials"), host.Scene.builtin("glass"), host.Scene.spheres(8, box=10.0, seed=3),
+                  host.Scene.field(12, seed=2, env_width=64)):
+        nodes, tris = hipcpu_wide.scene_arrays(scene.build())
+        assert hipcpu_wide.walk(lib, nodes, tris, _rays_through(np.random.default_rng(1), 10))[0] > 0
+
+
+def test_boxes_that_do_not_nest_are_left_to_the_binary_walk(lib):
+    """A caller's hierarchy in which an interior box is smaller than what lies below it: the binary walk misses triangles
+    outside of it. A wide node that leaves that box out would find them."""
+    rng = np.random.default_rng(4)
+    (nodes, tris), _ = _soup(rng, 1, 1)
+    rays = _rays_through(rng, 20000)
+    count, _, _, _ = hipcpu_wide.walk(lib, nodes, tris, rays)
+    assert count > 0
+    words = nodes.view(np.int32)
+    changed = 0
+    for i in range(1, min(40, len(nodes))):
+        for side in (0, 8):
+            if words[i, side + 7] == 0 and words[i, side + 3] >= 0:  # interior: the middle half of its box
+                lo, hi = nodes[i, side:side + 3].copy(), nodes[i, side + 4:side + 7].copy()
+                nodes[i, side:side + 3], nodes[i, side + 4:side + 7] = lo + (hi - lo) / 4, hi - (hi - lo) / 4
+                changed += 1
+    assert changed > 10
+    assert hipcpu_wide.walk(lib, nodes, tris, rays)[0] == 0
+
