@@ -1,0 +1,40 @@
+// Device memory of the wavefront engine's paths in flight: one entry per path slot in each array.
+#pragma once
+
+#include "internal.h"
+
+namespace phk {
+
+constexpr int kClasses = 4;  // shading queues (material classes)
+// Ordered compaction: a block of 256 threads covers 4096 slots, 16 consecutive slots per thread.
+constexpr int kCompactThreads = 256, kCompactPerThread = 16, kCompactChunk = kCompactThreads * kCompactPerThread;
+constexpr int kMaxCategories = 9;  // stages that one compaction tells apart
+
+inline int compact_chunks(int n) { return (n + kCompactChunk - 1) / kCompactChunk; }
+
+struct PathBuffers {
+    DevBuf<int> job, pixel, sample, sample_end, part, q_ext, q_shadow, q_term, q_miss, q_cls[kClasses], partial, first_pos;
+    DevBuf<uint8_t> stage;
+    DevBuf<uint64_t> rng;
+    DevBuf<float4> ro, rd, beta, L, hit, so, sd, sc;
+    int capacity = 0;  // slots that every array has room for
+
+    // Whether make_room(n) would allocate (what points into the arrays is to be dropped before).
+    bool moves(int n) const { return n != capacity; }
+
+    // Room for n slots. If an allocation fails there is room for none, and the next call allocates what is missing.
+    void make_room(int n) {
+        if (!moves(n)) return;
+        capacity = 0;
+        for (DevBuf<int>* b : {&job, &pixel, &sample, &sample_end, &part, &q_ext, &q_shadow, &q_term, &q_miss}) b->allocate(size_t(n));
+        for (auto& q : q_cls) q.allocate(size_t(n));
+        stage.allocate(size_t(n + 15) / 16 * 16);
+        partial.allocate(size_t(kMaxCategories) * size_t(compact_chunks(n)));
+        first_pos.allocate(size_t(kMaxCategories) * size_t(compact_chunks(n)));
+        rng.allocate(size_t(n));
+        for (DevBuf<float4>* b : {&ro, &rd, &beta, &L, &hit, &so, &sd, &sc}) b->allocate(size_t(n));
+        capacity = n;
+    }
+};
+
+}  // namespace phk

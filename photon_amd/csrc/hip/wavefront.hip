@@ -41,6 +41,7 @@
 #include <tuple>
 
 #include "device_scene.h"
+#include "path_buffers.h"
 #include "wavefront.h"
 
 using namespace phd;
@@ -74,8 +75,6 @@ PH_DEV uint8_t ext_stage(int bin) { return uint8_t(S_EXT | (bin << 3)); }
 // Bin of a continuing ray: its direction octant, or one shared bin when binning is off.
 PH_DEV int ray_bin(f3 d, int bins) { return bins ? 1 + (d.x < 0 ? 1 : 0) + (d.y < 0 ? 2 : 0) + (d.z < 0 ? 4 : 0) : 1; }
 
-constexpr int kClasses = 4;
-
 // Path state is read and written once per stage: streaming (non-temporal) accesses, so that it does not
 // push the BVH and triangle lines out of the caches.
 using v4f = float __attribute__((ext_vector_type(4)));
@@ -85,9 +84,6 @@ PH_DEV float4 ld_stream(const float4* p) {
 }
 PH_DEV void st_stream(float4* p, float4 a) { __builtin_nontemporal_store(v4f{a.x, a.y, a.z, a.w}, reinterpret_cast<v4f*>(p)); }
 constexpr int kMaxChunks = 1 << 16;
-// Ordered compaction: a block of 256 threads covers 4096 slots, 16 consecutive slots per thread.
-constexpr int kCompactThreads = 256, kCompactPerThread = 16, kCompactChunk = kCompactThreads * kCompactPerThread;
-constexpr int kMaxCategories = 9;
 
 struct JobParams {
     DScene scene;
@@ -1071,18 +1067,14 @@ std::vector<int> material_classes(const DScene& scene, hipStream_t st) {
     return cls;
 }
 
-struct WavefrontEngine::Impl {
+struct WavefrontEngine::Impl : PathBuffers {
     ph_wavefront_config cfg{128, 24, 0, 16, 1, 1, 16, 16, 0, 1, 1, 1, 10};
-    int slots = 0;
+    int slots = 0;  // of the running render or server
     int cus = 0;
-    DevBuf<int> job, pixel, sample, sample_end, part, counters, q_ext, q_shadow, q_term, q_miss, q_cls[kClasses], mat_class, partial, first_pos;
-    DevBuf<uint8_t> stage;
-    DevBuf<int> job_done;
+    DevBuf<int> counters, mat_class, job_done;
     DevBuf<long long> chunk_first;
     DevBuf<unsigned long long> items;  // next work item, items queued
     DevBuf<int4> chunk_pass;
-    DevBuf<uint64_t> rng;
-    DevBuf<float4> ro, rd, beta, L, hit, so, sd, sc;
     DevBuf<float4> part_sums;  // partial sums of a single render in sub-streams
     DevBuf<unsigned long long> direct_rays;  // direct_kernel's tallies
     DevBuf<JobParams> jobs;
@@ -1157,15 +1149,8 @@ struct WavefrontEngine::Impl {
     }
 
     void ensure_slots(int n) {
-        if (n == slots) return;
-        drop_graph();
-        for (DevBuf<int>* b : {&job, &pixel, &sample, &sample_end, &part, &q_ext, &q_shadow, &q_term, &q_miss}) b->allocate(size_t(n));
-        for (auto& q : q_cls) q.allocate(size_t(n));
-        stage.allocate(size_t(n + 15) / 16 * 16);
-        partial.allocate(size_t(kMaxCategories) * size_t(chunks_of(n)));
-        first_pos.allocate(size_t(kMaxCategories) * size_t(chunks_of(n)));
-        rng.allocate(size_t(n));
-        for (DevBuf<float4>* b : {&ro, &rd, &beta, &L, &hit, &so, &sd, &sc}) b->allocate(size_t(n));
+        if (moves(n)) drop_graph();
+        make_room(n);
         slots = n;
     }
 
@@ -1203,11 +1188,9 @@ struct WavefrontEngine::Impl {
         return f;
     }
 
-    static int chunks_of(int n) { return (n + kCompactChunk - 1) / kCompactChunk; }
-
     template <int Kind, bool Multi>
     void compact(hipStream_t st, const State& s) {
-        const int nch = chunks_of(slots);
+        const int nch = compact_chunks(slots);
         QueueOut out{};
         if (Kind == K_EXT) out.q[0] = s.q_ext;
         if (Kind == K_HIT) {

@@ -419,7 +419,15 @@ inline hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) {
 inline hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
 inline hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 inline hipError_t hipDeviceSynchronize() { return hipSuccess; }
+// Tests set how many more allocations succeed (negative: all of them).
+namespace hipcpu {
+inline int mallocs_left = -1, mallocs_made = 0;
+}
 inline hipError_t hipMalloc(void** p, size_t n) {
+    *p = nullptr;
+    if (hipcpu::mallocs_left == 0) return hipErrorOutOfMemory;
+    if (hipcpu::mallocs_left > 0) hipcpu::mallocs_left--;
+    hipcpu::mallocs_made++;
     *p = std::malloc(n ? n : 1);
     return *p ? hipSuccess : hipErrorOutOfMemory;
 }

@@ -1,0 +1,60 @@
+// The wavefront engine's path-state memory (photon_amd/csrc/hip/path_buffers.h) against allocations that fail.
+#include <cstdio>
+#include <cstdlib>
+
+#include "path_buffers.h"
+
+namespace phk {
+int set_error(const std::string&) { return -1; }
+}  // namespace phk
+
+using namespace phk;
+
+#define EXPECT(x)                                                   \
+    do {                                                            \
+        if (!(x)) {                                                 \
+            std::fprintf(stderr, "line %d: %s\n", __LINE__, #x);    \
+            std::exit(1);                                           \
+        }                                                           \
+    } while (0)
+
+static bool holds(const PathBuffers& b, size_t n) {
+    for (const DevBuf<int>* p : {&b.job, &b.pixel, &b.sample, &b.sample_end, &b.part, &b.q_ext, &b.q_shadow, &b.q_term, &b.q_miss})
+        if (!p->ptr || p->count < n) return false;
+    for (const DevBuf<int>& q : b.q_cls)
+        if (!q.ptr || q.count < n) return false;
+    for (const DevBuf<float4>* p : {&b.ro, &b.rd, &b.beta, &b.L, &b.hit, &b.so, &b.sd, &b.sc})
+        if (!p->ptr || p->count < n) return false;
+    const size_t chunks = size_t(kMaxCategories) * size_t(compact_chunks(int(n)));
+    return b.rng.ptr && b.rng.count >= n && b.stage.ptr && b.stage.count >= n && b.partial.ptr && b.partial.count >= chunks && b.first_pos.ptr &&
+           b.first_pos.count >= chunks;
+}
+
+// Every allocation of a growth fails in turn; the size that there was room for before is then asked for again.
+static void failed_growth() {
+    for (int fail = 0;; fail++) {
+        PathBuffers b;
+        b.make_room(5000);
+        EXPECT(holds(b, 5000));
+        hipcpu::mallocs_left = fail;
+        bool threw = false;
+        try {
+            b.make_room(20000);
+        } catch (const HipError&) {
+            threw = true;
+        }
+        hipcpu::mallocs_left = -1;
+        b.make_room(5000);
+        EXPECT(holds(b, 5000));
+        if (!threw) {
+            EXPECT(fail > 20);
+            return;
+        }
+    }
+}
+
+int main() {
+    failed_growth();
+    std::puts("ok");
+    return 0;
+}
