@@ -53,8 +53,27 @@ static void failed_growth() {
     }
 }
 
+// Sizes in turn allocate in the first round only; a size beyond the kept ones is given back.
+static void sizes_in_turn() {
+    PathBuffers b;
+    int first = 0;
+    for (int round = 0; round < 3; round++) {
+        for (int n : {4000, 16000, 48000}) {
+            b.make_room(n);
+            EXPECT(holds(b, size_t(n)));
+        }
+        if (round == 0) first = hipcpu::mallocs_made;
+    }
+    EXPECT(hipcpu::mallocs_made == first);
+    EXPECT(b.capacity == 48000);
+    b.capacity = PathBuffers::kKeptSlots + 1;  // as if so many had been asked for
+    b.make_room(4000);
+    EXPECT(b.capacity == 4000 && holds(b, 4000) && b.ro.count == 4000);
+}
+
 int main() {
     failed_growth();
+    sizes_in_turn();
     std::puts("ok");
     return 0;
 }

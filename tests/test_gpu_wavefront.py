@@ -182,3 +182,32 @@ def test_default_launch_at_every_size_keeps_the_image(name, w, h, spp, depth):
         r.close()
     assert planes[0] == planes[1]
     assert planes[0] == planes[2]
+
+
+def test_renders_of_changing_sizes_keep_their_images():
+    """Sample counts and launches in turn on one engine, whose path state stays: every image is the one that a
+    fresh engine renders, small renders after large ones too."""
+    scene = host.Scene.builtin("materials").build()
+    w, h = 640, 420
+    rs, cam = RenderSettings.make(w, h, max_depth=6, rr_depth=3, seed=4), scene.camera_view(w / h)
+    calls = [(1, {}), (5, {}), (12, {}), (5, {}), (4, dict(path_slots=3000)), (12, dict(path_slots=0)), (8, dict(path_slots=500000, sample_split=4)),
+             (5, dict(path_slots=0, sample_split=1)), (1, {}), (5, {})] + [(k, {}) for k in (5, 6, 7, 8, 9, 10, 11, 12, 13, 5)]
+
+    def image(r, spp, cfg):
+        if cfg:
+            r.set_wavefront_config(**cfg)
+        r.reset()
+        r.render(cam, rs, spp)
+        return gpu.copy_device_to_numpy(r.buffer_ptr(gpu.BUF_ACCUM), w * h * 16, np.float32).tobytes()
+
+    r = uploaded(scene, w, h, engine=gpu.ENGINE_WAVEFRONT)
+    state, fresh = {}, {}
+    for spp, cfg in calls:
+        state.update(cfg)
+        key = (spp, tuple(sorted(state.items())))
+        if key not in fresh:
+            one = uploaded(scene, w, h, engine=gpu.ENGINE_WAVEFRONT)
+            fresh[key] = image(one, spp, dict(state))
+            one.close()
+        assert image(r, spp, cfg) == fresh[key], (spp, state)
+    r.close()
