@@ -52,8 +52,9 @@ typedef struct ph_gpu_info {
 typedef struct ph_wavefront_config {
     int32_t block;         /* threads per block of the traversal kernels: 64, 128, 256 */
     int32_t stack_depth;   /* LDS stack entries per lane: 8, 16, 24, 32, 64 (rest spills to scratch) */
-    int32_t path_slots;    /* paths in flight (0: one per pixel, capped by memory; with sample_split 1 as well, the render's
-                              size decides: chunks of whole samples, each sample a work item, with the same image) */
+    int32_t path_slots;    /* paths in flight (0: one per pixel, at most 4M; with sample_split 1 as well, the render's size
+                              decides: chunks of whole samples, each sample a work item, over up to 8M paths (1.6 GB, and
+                              1 GB of partial sums; less where the device has less), with the same image) */
     int32_t blocks_per_cu; /* persistent grid: blocks per compute unit */
     int32_t sort_materials;/* shade in material-class queues */
     int32_t use_graph;     /* replay the bounce loop from a captured HIP graph */

@@ -16,6 +16,10 @@ namespace phk {
 struct HipError : std::runtime_error {
     using std::runtime_error::runtime_error;
 };
+// An allocation that the device's memory has no room for.
+struct OutOfMemory : HipError {
+    using HipError::HipError;
+};
 
 #define PH_CHECK(x)                                                                                               \
     do {                                                                                                          \
@@ -59,7 +63,9 @@ struct DevBuf {
         if (n == count && ptr) return;
         release();
         if (n == 0) return;
-        PH_CHECK(hipMalloc(reinterpret_cast<void**>(&ptr), n * sizeof(T)));
+        const hipError_t e = hipMalloc(reinterpret_cast<void**>(&ptr), n * sizeof(T));
+        if (e == hipErrorOutOfMemory) throw OutOfMemory(std::string("HIP error: ") + hipGetErrorString(e) + " (" + std::to_string(n * sizeof(T)) + " bytes)");
+        PH_CHECK(e);
         count = n;
     }
     // At least n elements: grows, never shrinks.

@@ -19,7 +19,7 @@ struct PathBuffers {
     DevBuf<float4> ro, rd, beta, L, hit, so, sd, sc;
     int capacity = 0;  // slots that every array has room for
 
-    // Renders of changing sizes keep the largest one's arrays, up to this many slots (1.8 GB): 1920x1080 Cornell with 1 and
+    // Renders of changing sizes keep the largest one's arrays, up to this many slots (1.6 GB): 1920x1080 Cornell with 1 and
     // 4 samples in turn takes 3.9 ms a pair, 16.4 with arrays of the exact size. What a configuration asked
     // for beyond that is given back by the next smaller call.
     static constexpr int kKeptSlots = 1 << 23;
@@ -39,6 +39,15 @@ struct PathBuffers {
         rng.allocate(size_t(n));
         for (DevBuf<float4>* b : {&ro, &rd, &beta, &L, &hit, &so, &sd, &sc}) b->allocate(size_t(n));
         capacity = n;
+    }
+
+    void release() {
+        capacity = 0;
+        for (DevBuf<int>* b : {&job, &pixel, &sample, &sample_end, &part, &q_ext, &q_shadow, &q_term, &q_miss, &partial, &first_pos}) b->release();
+        for (auto& q : q_cls) q.release();
+        stage.release();
+        rng.release();
+        for (DevBuf<float4>* b : {&ro, &rd, &beta, &L, &hit, &so, &sd, &sc}) b->release();
     }
 };
 

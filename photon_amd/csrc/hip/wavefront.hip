@@ -40,6 +40,7 @@
 #include <map>
 #include <tuple>
 
+#include "chunks.h"
 #include "device_scene.h"
 #include "path_buffers.h"
 #include "wavefront.h"
@@ -1154,6 +1155,12 @@ struct WavefrontEngine::Impl : PathBuffers {
         slots = n;
     }
 
+    void give_back() {
+        drop_graph();
+        release();
+        part_sums.release();
+    }
+
     State state() {
         State s;
         s.job = job.ptr;
@@ -1367,10 +1374,10 @@ ph_wavefront_config WavefrontEngine::config() const { return impl_->cfg; }
 // order, so the image is the in-order one bit for bit, and a chunk lasts as long as its longest paths, not as long as
 // the pixel with the longest run of them. 853x479, 8 samples of the materials scene: 3.5 ms, 11.8 with one item a
 // pixel; the 1M-triangle field's geometry at 1080p x 64 about 61 ms, 110 before. kChunkItems bounds the partial sums
-// (1 GB) and kChunkSlots the paths' state (1.7 GB; at 4M slots the field takes 68 ms). Two bounces a graph: a bounce
+// (1 GB) and kChunkSlots the paths' state (1.6 GB; at 4M slots the field takes 68 ms). Two bounces a graph: a bounce
 // that finds nothing costs 0.1 ms, a look at the queue 0.03. Chunks of at most kDirectItems samples run a sample per
 // lane: 64x64x4 Cornell box 0.32 ms (0.65 in bounces), 320x240x12 glass 1.56 (1.81), 640x360x4 materials 1.49 (2.1),
-// while 853x479x8 would take 4.4 against 3.5.
+// while 853x479x8 would take 4.4 against 3.5. Where memory is short, chunks get smaller (chunks.h).
 constexpr int64_t kChunkItems = int64_t(1) << 26, kChunkSlots = int64_t(1) << 23, kDirectItems = int64_t(1) << 20;
 constexpr int kChunkGraph = 2;
 
@@ -1390,18 +1397,19 @@ void WavefrontEngine::render(hipStream_t st, const WavefrontJob& job, bool count
         const int64_t slots = m.cfg.path_slots > 0 ? m.cfg.path_slots : std::min<int64_t>(pixels, 1 << 22);
         render_chunk(st, job, split, slots, m.cfg.graph_iterations, counting, stats);
     } else {
-        const int64_t chunks = (job.spp + std::max<int64_t>(1, kChunkItems / pixels) - 1) / std::max<int64_t>(1, kChunkItems / pixels);
-        for (int64_t c = 0; c < chunks; c++) {
-            const int k0 = int(c * job.spp / chunks), k1 = int((c + 1) * job.spp / chunks);
-            WavefrontJob part = job;
-            part.frame0 = job.frame0 + uint32_t(k0);
-            part.spp = k1 - k0;
-            if (k0 > 0) part.albedo = part.nd = nullptr;  // the first sample's
-            if (!counting && m.cfg.finish_percent > 0 && pixels * part.spp <= kDirectItems)
-                render_direct(st, part, stats);
-            else
-                render_chunk(st, part, part.spp, kChunkSlots, std::min(kChunkGraph, m.cfg.graph_iterations), counting, stats);
-        }
+        in_chunks(
+            pixels, job.spp, ChunkLimits{kChunkItems, kChunkSlots},
+            [&](int k0, int k1, int64_t slots) {
+                WavefrontJob part = job;
+                part.frame0 = job.frame0 + uint32_t(k0);
+                part.spp = k1 - k0;
+                if (k0 > 0) part.albedo = part.nd = nullptr;  // the first sample's
+                if (!counting && m.cfg.finish_percent > 0 && pixels * part.spp <= kDirectItems)
+                    render_direct(st, part, stats);
+                else
+                    render_chunk(st, part, part.spp, slots, std::min(kChunkGraph, m.cfg.graph_iterations), counting, stats);
+            },
+            [&] { m.give_back(); });
     }
     stats.extend_launches = stats.iterations;
     stats.shadow_launches = stats.iterations;

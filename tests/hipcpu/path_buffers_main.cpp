@@ -2,6 +2,7 @@
 #include <cstdio>
 #include <cstdlib>
 
+#include "chunks.h"
 #include "path_buffers.h"
 
 namespace phk {
@@ -71,7 +72,37 @@ static void sizes_in_turn() {
     EXPECT(b.capacity == 4000 && holds(b, 4000) && b.ro.count == 4000);
 }
 
+// A render in chunks where at most `room` slots and items fit: every sample runs once, in order, in chunks that fit.
+static void short_memory() {
+    for (int64_t pixels : {1, 7, 1000, 300000, 3000000})
+        for (int spp : {1, 2, 3, 64, 1000})
+            for (int64_t room : {int64_t(1) << 40, int64_t(1) << 22, int64_t(200000), kLeastSlots - 1}) {
+                int next = 0, failed = 0;
+                bool threw = false, released = true;
+                try {
+                    in_chunks(
+                        pixels, spp, ChunkLimits{int64_t(1) << 26, int64_t(1) << 23},
+                        [&](int k0, int k1, int64_t slots) {
+                            EXPECT(k0 == next && k1 > k0 && k1 <= spp && released);
+                            EXPECT(k1 - k0 == 1 || (k1 - k0) * pixels <= int64_t(1) << 26);
+                            if (std::min(slots, (k1 - k0) * pixels) > room) {
+                                failed++;
+                                released = false;
+                                throw OutOfMemory("no room");
+                            }
+                            next = k1;
+                        },
+                        [&] { released = true; });
+                } catch (const OutOfMemory&) {
+                    threw = true;
+                }
+                EXPECT(threw ? room < kLeastSlots : next == spp);
+                EXPECT(failed <= 8);
+            }
+}
+
 int main() {
+    short_memory();
     failed_growth();
     sizes_in_turn();
     std::puts("ok");

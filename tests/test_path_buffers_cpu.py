@@ -1,5 +1,5 @@
-"""The wavefront engine's path-state memory on the CPU (tests/hipcpu), under AddressSanitizer, with allocations that
-fail."""
+"""The wavefront engine's path-state memory and chunks on the CPU (tests/hipcpu), under AddressSanitizer, with allocations
+that fail."""
 import os
 import shutil
 import subprocess
@@ -13,7 +13,8 @@ import hipcpu_build  # noqa: E402
 
 def test_path_memory_after_failed_allocations(tmp_path):
     (tmp_path / "internal.h").write_text(hipcpu_build.internal_header())
-    shutil.copy(os.path.join(hipcpu_build.SRC, "path_buffers.h"), tmp_path)  # next to that internal.h
+    for header in ("path_buffers.h", "chunks.h"):
+        shutil.copy(os.path.join(hipcpu_build.SRC, header), tmp_path)  # next to that internal.h
     exe = str(tmp_path / "path_buffers")
     subprocess.run(["g++", "-std=c++20", "-O1", "-g", "-fsanitize=address,undefined", "-fno-sanitize-recover=undefined", "-pthread", f"-I{tmp_path}",
                     f"-I{os.path.join(HERE, 'hipcpu')}", f"-I{os.path.join(hipcpu_build.ROOT, 'include')}",
