@@ -51,16 +51,21 @@ typedef struct ph_gpu_info {
 /* Launch shape of the wavefront engine (chosen by ph_renderer_autotune or set explicitly). */
 typedef struct ph_wavefront_config {
     int32_t block;         /* threads per block of the traversal kernels: 64, 128, 256 */
-    int32_t stack_depth;   /* LDS stack entries per lane: 8, 16, 24, 32, 64 (rest spills to scratch) */
+    int32_t stack_depth;   /* LDS stack entries per lane: 8, 16, 24, 32, 64 (rest spills to scratch). Of the walk over the
+                              binary nodes: the four-wide nodes, which a render walks where the scene has them and
+                              lds_nodes is 0, take 12 whatever is set */
     int32_t path_slots;    /* paths in flight (0: one per pixel, at most 4M; with sample_split 1 as well, the render's size
                               decides: chunks of whole samples, each sample a work item, over up to 8M paths (1.6 GB, and
-                              1 GB of partial sums; less where the device has less), with the same image) */
+                              1 GB of partial sums; less where the device has less), with the same image. Up to 2^20
+                              samples such a render runs a sample per lane, unless finish_percent is 0 or counting
+                              is on, and looks at no other field; its rays are counted as rays_finish) */
     int32_t blocks_per_cu; /* persistent grid: blocks per compute unit */
     int32_t sort_materials;/* shade in material-class queues */
     int32_t use_graph;     /* replay the bounce loop from a captured HIP graph */
-    int32_t graph_iterations; /* bounces per captured graph */
+    int32_t graph_iterations; /* bounces per captured graph (at most 2 with path_slots 0 and sample_split 1) */
     int32_t refill_lanes;  /* a traversal wave takes new rays once this many of its 64 lanes are free */
-    int32_t lds_nodes;     /* top BVH nodes (breadth-first) each traversal block stages in LDS */
+    int32_t lds_nodes;     /* top binary BVH nodes (breadth-first) each traversal block stages in LDS; above 0, rays walk
+                              the binary nodes */
     int32_t ray_bins;      /* trace camera rays, then continuing rays by direction octant (1), or all together (0) */
     int32_t xcd_parts;     /* 8: each XCD takes a contiguous eighth of every queue (L2 locality); 1: all waves interleave */
     int32_t sample_split;  /* 1: all of a pixel's samples are added in order, and the accumulation is bit-identical
@@ -200,7 +205,8 @@ int ph_renderer_set_engine(ph_renderer* r, int engine);
 int ph_renderer_get_engine(const ph_renderer* r);
 int ph_renderer_set_wavefront_config(ph_renderer* r, const ph_wavefront_config* cfg);
 int ph_renderer_get_wavefront_config(const ph_renderer* r, ph_wavefront_config* cfg);
-/* Times candidate launch shapes on a short render of the given view and keeps the fastest. */
+/* Times candidate launch shapes on a short render of the given view and keeps the fastest. Fields that the render does not
+ * look at keep their values. */
 int ph_renderer_autotune(ph_renderer* r, const ph_camera_view* camera, const ph_render_settings* settings, int spp, ph_wavefront_config* chosen);
 int ph_renderer_set_counting(ph_renderer* r, int enable);
 int ph_renderer_stats(const ph_renderer* r, ph_render_stats* out);

@@ -1,4 +1,5 @@
-// A render in chunks of whole samples, as large as memory allows.
+// How a render runs for a launch configuration: the launch rule's sizes, renders in chunks of whole samples, as large as
+// memory allows, and which configurations run alike.
 #pragma once
 
 #include <algorithm>
@@ -33,6 +34,44 @@ void in_chunks(int64_t pixels, int spp, ChunkLimits limits, Run run, Release rel
             release();
         }
     }
+}
+
+// The rule of the default configuration (no path slots or sub-streams asked for), with its reasons at
+// WavefrontEngine::render.
+constexpr int64_t kChunkItems = int64_t(1) << 26, kChunkSlots = int64_t(1) << 23, kDirectItems = int64_t(1) << 20;
+constexpr int kChunkGraph = 2;
+
+inline bool default_launch(const ph_wavefront_config& c) { return c.sample_split == 1 && c.path_slots == 0; }
+
+// A render of at most kDirectItems samples at the default launch runs a sample per lane.
+inline bool runs_direct(const ph_wavefront_config& c, int64_t pixels, int spp) {
+    return default_launch(c) && c.finish_percent > 0 && pixels * spp <= kDirectItems;
+}
+
+// Sub-streams per pixel: the largest divisor of spp not above the configured split.
+inline int sub_streams(const ph_wavefront_config& c, int spp) {
+    int split = 1;
+    for (int k = 1; k <= std::min(c.sample_split, spp); k++)
+        if (spp % k == 0) split = k;
+    return split;
+}
+
+// The configuration with every field that this render does not look at set to one value: two configurations that give the
+// same here run the same launches.
+inline ph_wavefront_config effective_launch(ph_wavefront_config c, int64_t pixels, int spp, bool wide) {
+    if (runs_direct(c, pixels, spp)) {
+        c = ph_wavefront_config{};
+        c.sample_split = c.finish_percent = 1;
+        return c;
+    }
+    if (default_launch(c)) {
+        c.graph_iterations = std::min(c.graph_iterations, kChunkGraph);
+    } else {
+        c.sample_split = sub_streams(c, spp);
+        c.path_slots = int(std::min(c.path_slots > 0 ? int64_t(c.path_slots) : std::min<int64_t>(pixels, 1 << 22), pixels * c.sample_split));
+    }
+    if (wide && c.lds_nodes == 0) c.stack_depth = 0;  // the wide walk's stack has a depth of its own
+    return c;
 }
 
 }  // namespace phk

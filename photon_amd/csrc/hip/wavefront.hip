@@ -1378,9 +1378,6 @@ ph_wavefront_config WavefrontEngine::config() const { return impl_->cfg; }
 // that finds nothing costs 0.1 ms, a look at the queue 0.03. Chunks of at most kDirectItems samples run a sample per
 // lane: 64x64x4 Cornell box 0.32 ms (0.65 in bounces), 320x240x12 glass 1.56 (1.81), 640x360x4 materials 1.49 (2.1),
 // while 853x479x8 would take 4.4 against 3.5. Where memory is short, chunks get smaller (chunks.h).
-constexpr int64_t kChunkItems = int64_t(1) << 26, kChunkSlots = int64_t(1) << 23, kDirectItems = int64_t(1) << 20;
-constexpr int kChunkGraph = 2;
-
 void WavefrontEngine::render(hipStream_t st, const WavefrontJob& job, bool counting, ph_render_stats& stats) {
     Impl& m = *impl_;
     stats = ph_render_stats{};
@@ -1388,14 +1385,10 @@ void WavefrontEngine::render(hipStream_t st, const WavefrontJob& job, bool count
     const int64_t pixels = int64_t(job.width) * job.height;
     if (pixels <= 0 || job.spp <= 0) return;
     if (m.serving) throw std::runtime_error("the engine is serving; a progressive render needs its own engine");
-    if (m.cfg.sample_split != 1 || m.cfg.path_slots != 0) {
-        // Sub-streams per pixel: the largest divisor of spp not above the configured split.
-        int split = 1;
-        for (int k = 1; k <= std::min(m.cfg.sample_split, job.spp); k++)
-            if (job.spp % k == 0) split = k;
+    if (!default_launch(m.cfg)) {
         // Paths in flight: one per pixel up to a cap of 4M slots (~900 MB of state), unless told.
         const int64_t slots = m.cfg.path_slots > 0 ? m.cfg.path_slots : std::min<int64_t>(pixels, 1 << 22);
-        render_chunk(st, job, split, slots, m.cfg.graph_iterations, counting, stats);
+        render_chunk(st, job, sub_streams(m.cfg, job.spp), slots, m.cfg.graph_iterations, counting, stats);
     } else {
         in_chunks(
             pixels, job.spp, ChunkLimits{kChunkItems, kChunkSlots},
@@ -1404,7 +1397,7 @@ void WavefrontEngine::render(hipStream_t st, const WavefrontJob& job, bool count
                 part.frame0 = job.frame0 + uint32_t(k0);
                 part.spp = k1 - k0;
                 if (k0 > 0) part.albedo = part.nd = nullptr;  // the first sample's
-                if (!counting && m.cfg.finish_percent > 0 && pixels * part.spp <= kDirectItems)
+                if (!counting && runs_direct(m.cfg, pixels, part.spp))
                     render_direct(st, part, stats);
                 else
                     render_chunk(st, part, part.spp, slots, std::min(kChunkGraph, m.cfg.graph_iterations), counting, stats);
@@ -1534,7 +1527,14 @@ ph_wavefront_config WavefrontEngine::autotune(hipStream_t st, const WavefrontJob
     double best_ms = time_of(best);
     // A candidate replaces the current best only when it is faster by more than the run-to-run spread of
     // one render (about 1%), so that near-ties keep the earlier choice and repeated tunings agree.
+    // One that would run the same launches is not timed: its reading could only differ by that spread, and a field that
+    // this render does not look at would be kept for renders that do.
+    auto launch_of = [&](const ph_wavefront_config& c) {
+        return effective_launch(c, int64_t(job.width) * job.height, job.spp, job.scene.wide != nullptr);
+    };
     auto consider = [&](const ph_wavefront_config& c) {
+        const ph_wavefront_config a = launch_of(c), b = launch_of(best);
+        if (std::memcmp(&a, &b, sizeof(a)) == 0) return;
         const double t = time_of(c);
         if (t < best_ms * 0.98) best_ms = t, best = c;
     };

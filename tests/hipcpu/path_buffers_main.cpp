@@ -1,6 +1,8 @@
 // The wavefront engine's path-state memory (photon_amd/csrc/hip/path_buffers.h) against allocations that fail.
 #include <cstdio>
 #include <cstdlib>
+#include <cstring>
+#include <utility>
 
 #include "chunks.h"
 #include "path_buffers.h"
@@ -101,7 +103,49 @@ static void short_memory() {
             }
 }
 
+static bool alike(const ph_wavefront_config& a, const ph_wavefront_config& b, int64_t pixels, int spp, bool wide) {
+    const ph_wavefront_config x = effective_launch(a, pixels, spp, wide), y = effective_launch(b, pixels, spp, wide);
+    return std::memcmp(&x, &y, sizeof(x)) == 0;
+}
+
+// Which configurations the tuner may not tell apart.
+static void same_launches() {
+    const ph_wavefront_config base{128, 24, 0, 16, 1, 1, 16, 16, 0, 1, 1, 1, 10};
+    using Field = int32_t ph_wavefront_config::*;
+    const std::pair<Field, int> changes[] = {{&ph_wavefront_config::block, 64},          {&ph_wavefront_config::stack_depth, 8},
+                                             {&ph_wavefront_config::blocks_per_cu, 4},   {&ph_wavefront_config::refill_lanes, 32},
+                                             {&ph_wavefront_config::ray_bins, 0},        {&ph_wavefront_config::xcd_parts, 8},
+                                             {&ph_wavefront_config::lds_nodes, 128},     {&ph_wavefront_config::use_graph, 0},
+                                             {&ph_wavefront_config::graph_iterations, 8}, {&ph_wavefront_config::finish_percent, 30}};
+    for (const auto& [field, value] : changes) {
+        ph_wavefront_config c = base;
+        c.*field = value;
+        EXPECT(alike(base, c, 1 << 18, 4, true) && alike(base, c, 1 << 18, 4, false));  // a sample per lane: nothing is looked at
+        const bool depth = field == &ph_wavefront_config::stack_depth, graph = field == &ph_wavefront_config::graph_iterations;
+        EXPECT(alike(base, c, 1 << 18, 5, true) == (depth || graph));
+        EXPECT(alike(base, c, 1 << 18, 5, false) == graph);
+        ph_wavefront_config slots = base, slots_c = c;
+        slots.path_slots = slots_c.path_slots = 100000;
+        EXPECT(alike(slots, slots_c, 1 << 18, 4, true) == depth);
+        EXPECT(!alike(slots, slots_c, 1 << 18, 4, false));
+        slots.lds_nodes = 64;  // the binary nodes' top in LDS: over the binary nodes
+        slots_c.lds_nodes = std::max(64, slots_c.lds_nodes);
+        EXPECT(!alike(slots, slots_c, 1 << 18, 4, true));
+    }
+    ph_wavefront_config c = base, d = base;
+    c.finish_percent = 0;  // in bounces
+    EXPECT(!alike(base, c, 1 << 18, 4, true));
+    c = base;
+    c.path_slots = 1 << 18, d.path_slots = 1 << 20;  // no more slots than items
+    EXPECT(alike(c, d, 1 << 18, 4, true) && !alike(c, base, 1 << 18, 4, true));
+    c.sample_split = 4, d.sample_split = 5;  // rounded down to a divisor
+    EXPECT(!alike(c, d, 1 << 18, 4, true));  // now there are items for the slots
+    d.path_slots = c.path_slots;
+    EXPECT(alike(c, d, 1 << 18, 4, true) && !alike(c, d, 1 << 18, 20, true));
+}
+
 int main() {
+    same_launches();
     short_memory();
     failed_growth();
     sizes_in_turn();

@@ -211,3 +211,27 @@ def test_renders_of_changing_sizes_keep_their_images():
             one.close()
         assert image(r, spp, cfg) == fresh[key], (spp, state)
     r.close()
+
+
+@pytest.mark.parametrize("w,h,spp", [(64, 64, 2), (512, 512, 5)])
+def test_autotune_changes_only_what_the_render_looks_at(w, h, spp):
+    """A render that runs a sample per lane (64 x 64 x 2) looks at no field but those that lead it elsewhere, so tuning it
+    cannot change the others; a render in bounces over wide nodes looks at neither stack depth nor, at the default launch,
+    long graphs. The tuned image is the untuned one where the samples are added in order."""
+    scene = host.Scene.builtin("cornell-c1").build()
+    rs, cam = RenderSettings.make(w, h, max_depth=4, rr_depth=3, seed=2), scene.camera_view(w / h)
+    r = uploaded(scene, w, h, engine=gpu.ENGINE_WAVEFRONT)
+    before = r.wavefront_config().as_dict()
+    r.render(cam, rs, spp)
+    image = r.download_image()
+    cfg = r.autotune(cam, rs, spp).as_dict()
+    if cfg["path_slots"] == 0 and cfg["sample_split"] == 1:
+        if w * h * spp <= 1 << 20 and cfg["finish_percent"] > 0:
+            assert cfg == before
+        assert cfg["graph_iterations"] <= 2 or cfg["graph_iterations"] == before["graph_iterations"]
+    assert cfg["lds_nodes"] > 0 or cfg["stack_depth"] == before["stack_depth"]
+    r.reset()
+    r.render(cam, rs, spp)
+    if spp % cfg["sample_split"] or cfg["sample_split"] in (1, spp):
+        assert r.download_image().tobytes() == image.tobytes()
+    r.close()
