@@ -207,8 +207,10 @@ __global__ __launch_bounds__(kRowX* kRowY) void temporal_kernel(In in, ph_camera
     const float variance = fmaxf(0.0f, m1 - m0 * m0);
     out_illum[i] = make_float4(c.x, c.y, c.z, len);
     out_moments[i] = make_float4(m0, m1, variance, 0.0f);
-    out_filter[i] = make_float4(c.x, c.y, c.z, variance);
-    if (len < 4.0f && mat >= 0) short_history[block] = 1;
+    if (len < 4.0f && mat >= 0)
+        short_history[block] = 1;  // the variance pass writes this pixel (a first 1600x900 frame: 0.340 ms with both writing it, 0.336)
+    else
+        out_filter[i] = make_float4(c.x, c.y, c.z, variance);
 }
 
 // The 7x7 estimate of one short-history pixel (svgf.cu:96-132): moments and illumination of the taps
