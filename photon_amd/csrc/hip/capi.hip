@@ -572,18 +572,24 @@ int ph_trace(ph_renderer* r, const ph_ray* rays, int n, int anyhit, ph_hit* hits
     if (!r->uploaded) return fail("no scene uploaded");
     return guarded([&] {
         ph_renderer& m = *r;
-        // Closest hits do not depend on the walk (dwide.h names the exception), so they go over the wide nodes. Any-hit results are the first hit of
-        // the binary walk's order, and counts are its counts. Any-hit rays end at very different times: with more than
-        // one and a half rays for each of the chip's 524,288 lanes a fixed grid with refilled lanes is faster
-        // (1,000,003 rays into 16K / 64K / 256K triangles 0.33 / 0.48 / 0.50 ms in blocks, 0.31 / 0.43 / 0.49 refilled;
-        // 4M rays 1.07 / 1.54 / 1.62, 0.79 / 1.24 / 1.52), below that the blocks are (250,000: 0.13 / 0.16 / 0.18, 0.15 /
-        // 0.18 / 0.20). Asking the wide nodes first whether anything is hit cost more than it saved (0.73 ms, 84 %
-        // of 1,000,003 rays hitting).
-        constexpr int kRefillRays = 3 << 18;
-        const bool refill = anyhit && !counts && n >= kRefillRays;
+        // Closest hits do not depend on the walk (dwide.h names the exception), so they go over the wide nodes. Any-hit
+        // results are the first hit of the binary walk's order, and counts are its counts.
+        // Any-hit launches, ms for shadow / camera / random / short rays into 64K triangles (16K and 256K alike):
+        //   * 128-ray blocks with 32-entry stacks, 5 waves per SIMD, up to three quarters of a million rays;
+        //   * from there on with 16-entry stacks, 8 waves. 1,000,003 rays: 0.46 / 0.126 / 0.160 / 0.056 with 32 entries, 0.38 /
+        //     0.126 / 0.137 / 0.052 with 16. Below, camera rays ran slower that way (600,000: 0.114 against 0.122);
+        //   * from nearly four rays for each of the chip's 524,288 lanes on, a grid with refilled lanes, for rays that end at
+        //     very different times. 2M: 0.81 / 0.174 / 0.250 / 0.084 with 32 entries, 0.63 / 0.150 / 0.202 / 0.071 with 16, 0.66 /
+        //     0.174 / 0.144 / 0.065 refilled; 4M: 1.51 / 0.257 / 0.442 / 0.138, 1.15 / 0.208 / 0.327 / 0.111, 1.20 / 0.234 / 0.187 /
+        //     0.086. Camera rays, which end together, lose by it: slightly there (16K triangles, 2M: 0.119 with 32 entries,
+        //     0.123), below it too much (64K, 1,000,003: 0.142).
+        // Asking the wide nodes first whether anything is hit cost more than it saved (0.73 ms, 84 % of 1,000,003 rays
+        // hitting).
+        constexpr int kShortStackRays = 3 << 18, kRefillRays = 15 << 17;
+        const bool many = anyhit && !counts && n >= kShortStackRays, refill = many && n >= kRefillRays;
         if (m.view.wide && !anyhit && !counts)
             launch_trace_wide(m.stream, m.view, rays, n, hits);
-        else if (!launch_trace(m.stream, m.view, rays, n, anyhit != 0, hits, counts, refill ? 256 : 128, refill ? 16 : 32, refill, 0, refill ? 2048 : 0))
+        else if (!launch_trace(m.stream, m.view, rays, n, anyhit != 0, hits, counts, 128, many ? 16 : 32, refill, 0, refill ? 4096 : 0))
             return fail("unsupported traversal launch shape");
         PH_CHECK(hipStreamSynchronize(m.stream));
         return 0;

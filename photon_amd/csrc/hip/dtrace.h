@@ -303,7 +303,7 @@ PH_DEV void trace_stream(int n, int parts, int refill, TraceScene ts, Stack& sta
         bool live = false;
         int ray = -1;  // this lane's; -2 - ray once it is to be traced again
         for (;;) {
-            const uint64_t free = __ballot(!live && ray >= -1);
+            const uint64_t free = __ballot(!live && (!Walk::kSecond || ray >= -1));
             const bool none = __ballot(live) == 0;
             if (none || (!drained && __popcll(free) >= refill)) {
                 if (!live && ray >= 0) {

@@ -228,13 +228,18 @@ __global__ __launch_bounds__(Block) void trace_kernel(DScene s, const ph_ray* ra
     LaneStack<Depth> stack{lds + threadIdx.x, Block, spill.v};
     if (Persistent) {
         // A fixed grid; each wave refills its lanes from its share of the rays (trace_stream), with the
-        // top of the tree staged in LDS.
+        // top of the tree staged in LDS if asked for. Without, no step looks there: 4M any-hit rays into 262,144
+        // triangles 1.59 -> 1.56 ms from all directions, 0.42 -> 0.39 from a camera.
         TraceScene ts = trace_scene(s);
-        ts.top = top_nodes;
-        ts.top_n = min(lds_nodes, s.top_nodes);
-        stage_top_nodes(top_nodes, s.nodes, ts.top_n);
         BinaryWalk<AnyHit, false> walk{};
-        trace_rays<AnyHit>(rays, n, 16, ts, stack, walk, hits);
+        if (lds_nodes == 0) {
+            trace_rays<AnyHit>(rays, n, 16, ts, stack, walk, hits);
+        } else {
+            ts.top = top_nodes;
+            ts.top_n = min(lds_nodes, s.top_nodes);
+            stage_top_nodes(top_nodes, s.nodes, ts.top_n);
+            trace_rays<AnyHit>(rays, n, 16, ts, stack, walk, hits);
+        }
     } else {
         const int i = blockIdx.x * Block + threadIdx.x;
         if (i < n) trace_one(s, rays, i, AnyHit, hits, counts, stack, Tag<Count>{}, Tag<AnyHit>{});

@@ -128,10 +128,10 @@ def test_wavefront_image_over_either_walk(w, h, spp, split):
     r.close()
 
 
-@pytest.mark.parametrize("n", [1, 129, 786431, 786432, 1000003])
+@pytest.mark.parametrize("n", [1, 129, 786431, 786432, 1000003, 1966079, 1966080, 2500007])
 def test_any_hit_launches_report_the_same_hits(n):
-    """Few any-hit rays run in blocks, many (from 786,432 on) in a grid with refilled lanes: both report the counting
-    walk's hits."""
+    """Few any-hit rays run in blocks with deep stacks, more (from 786,432 on) in blocks with short ones, many (from 1,966,080
+    on) in a grid with refilled lanes: all report the counting walk's hits."""
     scene = host.Scene.spheres(12, box=12.0, alpha_fraction=0.3, seed=4).build()
     r = uploaded(scene)
     rays = scene.shadow_rays(n, seed=3)
