@@ -56,7 +56,7 @@ public:
     bool ready() const { return ready_; }
     size_t bytes() const {
         size_t b = 0;
-        b += nodes_.bytes() + wide_.bytes() + tris_.bytes() + materials_.bytes() + indices_.bytes() + tri_emissive_.bytes();
+        b += nodes_.bytes() + wide_.nodes.bytes() + tris_.bytes() + materials_.bytes() + indices_.bytes() + tri_emissive_.bytes();
         b += normals_.bytes() + uvs_.bytes() + tangents_.bytes() + srgb_lut_.bytes() + env_texels_.bytes();
         b += env_marginal_.bytes() + env_conditional_.bytes() + textures_.bytes() + texels_.bytes();
         b += guide_marginal_.bytes() + guide_conditional_.bytes() + env_trig_.bytes();
@@ -83,6 +83,11 @@ public:
         const std::vector<ph_bvh_node> relabelled = relabel_top_first(d.nodes, d.num_nodes, kTopNodes, top);
         nodes_.upload(relabelled.data(), size_t(d.num_nodes) * 4, st);
         PH_CHECK(hipStreamSynchronize(st));  // the host copy above goes out of scope
+        try {  // runs while the arrays below are copied
+            build_wide_nodes(st, nodes_.ptr, d.num_nodes, d.num_tris, wide_);
+        } catch (const OutOfMemory&) {
+            (void)hipGetLastError();  // the scene is traced over the binary nodes
+        }
         indices_.upload(d.indices, size_t(d.num_tris) * 3, st);
         normals_.upload(d.normals, d.normals ? size_t(d.num_vertices) * 3 : 0, st);
         uvs_.upload(d.uvs, d.uvs ? size_t(d.num_vertices) * 2 : 0, st);
@@ -95,8 +100,6 @@ public:
         v.nodes = or_null(nodes_);
         v.num_nodes = d.num_nodes;
         upload_lights(d, st);
-        build_wide_nodes(st, nodes_.ptr, d.num_nodes, d.num_tris, wide_);
-        v.wide = or_null(wide_);
         v.indices = or_null(indices_);
         v.normals = or_null(normals_);
         v.uvs = or_null(uvs_);
@@ -112,6 +115,7 @@ public:
         float dx = d.bounds_max[0] - d.bounds_min[0], dy = d.bounds_max[1] - d.bounds_min[1], dz = d.bounds_max[2] - d.bounds_min[2];
         extent_ = std::fmax(std::sqrt(dx * dx + dy * dy + dz * dz), 1e-3f);
         PH_CHECK(hipStreamSynchronize(st));
+        v.wide = wide_.settled();
         ready_ = true;
     }
 
@@ -174,7 +178,8 @@ public:
     }
 
 private:
-    DevBuf<float4> nodes_, wide_, tris_, materials_;
+    DevBuf<float4> nodes_, tris_, materials_;
+    WideNodes wide_;
     DevBuf<int> indices_, tri_emissive_;
     DevBuf<float> env_trig_, normals_, uvs_, tangents_, srgb_lut_, env_texels_, env_marginal_, env_conditional_;
     DevBuf<int> guide_marginal_, guide_conditional_;

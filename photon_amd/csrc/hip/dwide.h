@@ -15,7 +15,7 @@
 //   [0]  origin.xyz, three signed exponent bytes: plane q of an axis lies at origin + q 2^exponent
 //   [1]  lower x, upper x, lower y, upper y planes of the four children, a byte each
 //   [2]  lower z, upper z, and two unused words
-//   [3]  four links: interior (a wide node's index, >= 0) or leaf (bit 31, 5 bits triangles - 1, 26 bits
+//   [3]  four links: interior (a wide node's index, its binary node's, >= 0) or leaf (bit 31, 5 bits triangles - 1, 26 bits
 //        first triangle). An unused child has an inverted box and a sibling's link.
 //
 // The answer is the binary walk's, with the one exception below:

@@ -435,6 +435,9 @@ inline hipError_t hipFree(void* p) {
     std::free(p);
     return hipSuccess;
 }
+constexpr unsigned hipHostMallocDefault = 0;
+inline hipError_t hipHostMalloc(void** p, size_t n, unsigned) { return hipMalloc(p, n); }
+inline hipError_t hipHostFree(void* p) { return hipFree(p); }
 inline hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind, hipStream_t) {
     if (n) std::memcpy(d, s, n);
     return hipSuccess;

@@ -38,7 +38,7 @@ def scene_arrays(scene):
 
 
 def walk(lib, nodes, tris, rays, anyhit=False):
-    """(wide nodes, binary hits, wide hits, traced again) of every ray."""
+    """(whether there are wide nodes, binary hits, wide hits, traced again) of every ray."""
     rays = np.ascontiguousarray(rays, RAY_DTYPE)
     n = len(rays)
     hits, again = np.zeros((n, 2), HIT_DTYPE), np.zeros(n, np.int32)

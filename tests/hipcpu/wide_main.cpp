@@ -58,16 +58,18 @@ void one_ray(const TraceScene& ts, const float* r, HitRec* out, int* again) {
 }  // namespace
 
 // Each ray (7 floats) over both kinds of nodes: hits[2 i] the binary walk's, hits[2 i + 1] the wide walk's; again[i]:
-// the wide walk left the ray to the binary one. Returns the number of wide nodes, 0 if the scene has none.
+// the wide walk left the ray to the binary one. Returns 0 if the scene has no wide nodes.
 extern "C" __attribute__((visibility("default"))) int walk_both(const float* nodes, int num_nodes, const float* tris, int num_tris, const float* rays, int n, int anyhit, HitRec* hits, int* again) {
-    phk::DevBuf<float4> wide, dev_nodes, dev_tris;
+    phk::DevBuf<float4> dev_nodes, dev_tris;
+    phk::WideNodes wide;
     dev_nodes.upload(nodes, size_t(num_nodes) * 4, nullptr);
     dev_tris.upload(tris, size_t(num_tris) * 3, nullptr);
-    if (!phk::build_wide_nodes(nullptr, dev_nodes.ptr, num_nodes, num_tris, wide)) return 0;
+    phk::build_wide_nodes(nullptr, dev_nodes.ptr, num_nodes, num_tris, wide);
+    if (!wide.settled()) return 0;
     phk::mark_leaves(nullptr, dev_nodes.ptr, num_nodes, num_tris, dev_tris.ptr);
     DScene s{};
     s.nodes = dev_nodes.ptr;
-    s.wide = wide.ptr;
+    s.wide = wide.nodes.ptr;
     s.tris = dev_tris.ptr;
     s.num_nodes = num_nodes;
     s.num_tris = num_tris;
@@ -82,5 +84,5 @@ extern "C" __attribute__((visibility("default"))) int walk_both(const float* nod
     for (int k = 1; k < 8; k++) pool.emplace_back(work);
     work();
     for (std::thread& t : pool) t.join();
-    return int(wide.count / 4);
+    return num_nodes;
 }
