@@ -61,6 +61,10 @@ struct Job {
 // A finished job's image: each pixel's partial sums in sub-stream order (one: the accumulation itself), over the
 // samples. On the device: the host's sum read all 16-byte partial sums over the bus, into fresh pages (eight jobs of
 // 65K to 921K pixels: 25 ms, 5 ms with this kernel and the 12-byte pixels copied).
+// An image is read in pieces of kResultPixels, through a buffer that the server has from the start: a result needs no memory
+// that other work may have taken, whatever its size.
+constexpr int kResultPixels = 1 << 20;
+
 __global__ __launch_bounds__(256) void resolve_kernel(const float4* sums, int pixels, int split, float inv, float* rgb) {
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= pixels) return;
@@ -99,7 +103,7 @@ struct ph_server {
     Lane lanes[2];  // 0: main, 1: express
     std::vector<std::unique_ptr<ServedScene>> scenes;
     std::vector<std::unique_ptr<Job>> jobs;
-    DevBuf<float> image;  // the result being read: as large as the largest read so far
+    DevBuf<float> piece;  // of the result being read
     int64_t mem_used = 0;
     int finished = 0;
     std::chrono::steady_clock::time_point t0 = std::chrono::steady_clock::now();
@@ -122,6 +126,7 @@ struct ph_server {
         if (cfg.express_samples <= 0) cfg.express_samples = int64_t(16) * cfg.express_slots;
         if (cfg.express_iterations <= 0) cfg.express_iterations = cfg.iterations_per_step;
         PH_CHECK(hipGetDevice(&device));
+        piece.allocate(3 * size_t(kResultPixels));
         const int slots[2] = {cfg.path_slots, cfg.express_slots};
         for (int k = 0; k < 2; k++) {
             Lane& L = lanes[k];
@@ -390,18 +395,38 @@ int ph_server_status(const ph_server* s, int job, ph_job_status* out) {
     return 0;
 }
 
+namespace {
+
+// Kernels are launched on the server's GPU whatever the calling thread's current one is (a result may be read by another
+// thread than the one that runs the server).
+struct OnDevice {
+    int before = 0, device;
+    explicit OnDevice(int d) : device(d) {
+        PH_CHECK(hipGetDevice(&before));
+        if (before != device) PH_CHECK(hipSetDevice(device));
+    }
+    ~OnDevice() {
+        if (before != device) (void)hipSetDevice(before);
+    }
+};
+
+}  // namespace
+
 int ph_server_result(ph_server* s, int job, float* rgb) {
     if (!s || !rgb) return set_error("null argument");
     if (job < 0 || job >= int(s->jobs.size())) return set_error("unknown job id");
     Job& j = *s->jobs[size_t(job)];
     if (j.status.state != PH_JOB_DONE) return set_error(j.status.state == PH_JOB_RELEASED ? "the job's result was already read" : "the job is not done");
     return guarded([&] {
+        const OnDevice gpu(s->device);
         const size_t n = size_t(j.status.pixels);
-        s->image.reserve(3 * n);
-        hipLaunchKernelGGL(resolve_kernel, dim3(unsigned((n + 255) / 256)), dim3(256), 0, s->stream(), j.accum.ptr, j.status.pixels, j.split,
-                           1.0f / float(j.desc.spp), s->image.ptr);
-        PH_CHECK(hipGetLastError());
-        PH_CHECK(hipMemcpyAsync(rgb, s->image.ptr, 3 * n * sizeof(float), hipMemcpyDeviceToHost, s->stream()));
+        for (size_t i = 0; i < n; i += kResultPixels) {
+            const int m = int(std::min<size_t>(kResultPixels, n - i));
+            hipLaunchKernelGGL(resolve_kernel, dim3((m + 255) / 256), dim3(256), 0, s->stream(), j.accum.ptr + i * size_t(j.split), m, j.split,
+                               1.0f / float(j.desc.spp), s->piece.ptr);
+            PH_CHECK(hipGetLastError());
+            PH_CHECK(hipMemcpyAsync(rgb + 3 * i, s->piece.ptr, 3 * size_t(m) * sizeof(float), hipMemcpyDeviceToHost, s->stream()));
+        }
         PH_CHECK(hipStreamSynchronize(s->stream()));
         j.accum.release();
         s->mem_used -= int64_t(j.bytes);

@@ -150,3 +150,32 @@ def test_errors():
     with pytest.raises(RuntimeError, match="already"):
         srv.result(j)
     srv.close()
+
+
+@pytest.mark.parametrize("w,h,min_items", [(1024, 1024, 1), (1025, 1024, 1), (1500, 1600, 1), (1500, 1600, 9000000)])
+def test_results_are_read_in_pieces(scenes, w, h, min_items):
+    """Images of exactly one piece (2^20 pixels), a little more, and several, with one partial sum a pixel and with one a
+    sample."""
+    job = ("cornell-c1", w, h, 4, 3, 7)
+    got = _serve(scenes, [job], [0], path_slots=1 << 20, min_items=min_items, express_slots=-1)[0]
+    assert got.tobytes() == _alone(scenes["cornell-c1"], w, h, 4, 3, 7).tobytes()
+
+
+def test_a_large_result_leaves_no_memory_behind(scenes):
+    """What the server holds after a large result was read is what it held before the job: 4096 x 4096 pixels are 192 MiB
+    as an image."""
+    import torch
+
+    srv = gpu.Server(path_slots=1 << 18, express_slots=-1)
+    sid = srv.add_scene(scenes["furnace"])
+
+    def serve(w, h):
+        j = srv.submit(sid, w, h, 1, scenes["furnace"].camera_view(w / h), max_depth=1, seed=1)
+        srv.run_until_idle()
+        assert np.isfinite(srv.result(j)).all()
+
+    serve(64, 64)
+    before = torch.cuda.mem_get_info()[0]
+    serve(4096, 4096)
+    assert before - torch.cuda.mem_get_info()[0] < 64 << 20
+    srv.close()
