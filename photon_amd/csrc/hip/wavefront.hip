@@ -1090,13 +1090,13 @@ struct WavefrontEngine::Impl : PathBuffers {
     std::vector<hipEvent_t> events;
     hipGraphExec_t graph_exec = nullptr;
     std::tuple<int, int, int, int, int, bool, bool> graph_key{};
-    bool wide = false;  // every scene in work has wide nodes
+    bool wide = false;  // rays walk the wide nodes, which every scene in work has
     std::map<std::tuple<const void*, int, int, int, int>, ph_wavefront_config> tuned;
     // Serving bookkeeping (host side).
     bool serving = false;
     std::vector<bool> entry_used;
     std::vector<int> entry_pixels;
-    std::vector<bool> entry_wide;
+    std::vector<int> entry_nodes;  // 0: no wide nodes
     // A queued pass: its unstarted items are [next, pixels) of the job's pixel order. While laid out,
     // its items occupy the segments (first, length) of the item index space, in pixel order: one
     // segment for a contiguous layout, one per round for a round-robin one.
@@ -1131,7 +1131,7 @@ struct WavefrontEngine::Impl : PathBuffers {
         cus = device_cus();
         entry_used.assign(kMaxJobs, false);
         entry_pixels.assign(kMaxJobs, 0);
-        entry_wide.assign(kMaxJobs, false);
+        entry_nodes.assign(kMaxJobs, 0);
     }
     ~Impl() {
         drop_graph();
@@ -1220,10 +1220,12 @@ struct WavefrontEngine::Impl : PathBuffers {
     void iteration(hipStream_t st, const ShapeFns& fns, bool count, hipEvent_t* ev) {
         // Traversal: what fits the chip at once, or over the wide nodes four times that. The shares of a wave cost very
         // differently, and blocks that start as others end even them out (1080p, 64 samples, 1M triangles: 79.0 ms,
-        // 83.0 with one round of blocks, 81.1 with two). Never more lanes than slots: a queue holds no more.
+        // 83.0 with one round of blocks, 81.1 with two). Serving takes one round: its queues are often short, and blocks that
+        // find nothing cost it more (1280x720x4 Cornell job 2.80 ms, 2.84 with four; the mixed stream 26.2 either way).
+        // Never more lanes than slots: a queue holds no more.
         const auto blocks_for = [&](int most, int block) { return std::max(1, std::min(most, (slots + block - 1) / block)); };
         const bool over_wide = wide && !count && (Multi || cfg.lds_nodes == 0);
-        const int tgrid = blocks_for(cus * std::max(1, cfg.blocks_per_cu) * (over_wide ? 4 : 1), cfg.block);
+        const int tgrid = blocks_for(cus * std::max(1, cfg.blocks_per_cu) * (over_wide && !Multi ? 4 : 1), cfg.block);
         // Shading: 4 blocks of 256 threads per CU, all of them resident: the shading kernels need 140 VGPRs since the
         // bounded trigonometry (dtrig.h; 232 before, 2 waves per SIMD), and 128 spill at most 8. 1080p, 64 samples, 1M
         // triangles: 79.6 ms at 3 waves per SIMD, 75.0 at 4, 78.4 at 5; 8 to 32 blocks per CU 74.4 to 75.0.
@@ -1655,7 +1657,7 @@ int WavefrontEngine::serve_admit(hipStream_t st, const WavefrontJob& job) {
     PH_CHECK(hipMemsetAsync(m.job_done.ptr + entry, 0, sizeof(int), st));
     m.host_done[entry] = 0;
     m.entry_used[size_t(entry)] = true;
-    m.entry_wide[size_t(entry)] = job.scene.wide != nullptr;
+    m.entry_nodes[size_t(entry)] = job.scene.wide ? job.scene.num_nodes : 0;
     m.entry_pixels[size_t(entry)] = job.width * job.height * job.split;
     return entry;
 }
@@ -1683,6 +1685,13 @@ void WavefrontEngine::serve_share(int quantum) {
     impl_->share_quantum = std::max(0, quantum);
     impl_->chunks_dirty = true;
 }
+
+// Serving walks the binary nodes if a scene in work has no others, and if all have few: each bounce waits for its longest
+// rays, and where a walk is short the wide one's longer steps make those longer. Jobs of 64x64x1 / 1280x720x4 over wide and
+// over binary nodes: 17 nodes (Cornell box) 1.12 / 3.59 ms and 1.02 / 3.33; 247 nodes 0.83 / 2.25 and 0.81 / 2.23; 996 nodes
+// 0.91 / 2.52 and 0.89 / 2.55; 3,968 nodes 1.00 / 2.91 and 0.99 / 2.99. (Renders at the default launch are faster over wide
+// nodes at every size.)
+constexpr int kFewNodes = 512;
 
 void WavefrontEngine::serve_run(hipStream_t st, int iterations) {
     Impl& m = *impl_;
@@ -1753,9 +1762,13 @@ void WavefrontEngine::serve_run(hipStream_t st, int iterations) {
     }
     m.passes.swap(keep);
     m.chunks_dirty = false;
-    m.wide = true;
+    int least = INT32_MAX, most = 0;
     for (int e = 0; e < kMaxJobs; e++)
-        if (m.entry_used[size_t(e)] && !m.entry_wide[size_t(e)]) m.wide = false;
+        if (m.entry_used[size_t(e)]) {
+            least = std::min(least, m.entry_nodes[size_t(e)]);
+            most = std::max(most, m.entry_nodes[size_t(e)]);
+        }
+    m.wide = least > 0 && most > kFewNodes;
     m.run_batch(st, std::max(1, iterations), true, false);
     PH_CHECK(hipMemcpyAsync(m.host_done, m.job_done.ptr, kMaxJobs * sizeof(int), hipMemcpyDeviceToHost, st));
     PH_CHECK(hipStreamSynchronize(st));
