@@ -9,7 +9,7 @@ import numpy as np
 from photon_amd.types import NODE_DTYPE
 
 
-def run(exe, positions, indices, threads=8, timeout=None):
+def run(exe, positions, indices, threads=8, timeout=None, max_leaf=8, traversal_cost=1.0):
     """Returns (nodes, order, stats bytes, wall seconds) of the build of `positions` (V, 3) float32 and
     `indices` (T, 3) int32."""
     p = np.ascontiguousarray(positions, np.float32).reshape(-1, 3)
@@ -24,7 +24,7 @@ def run(exe, positions, indices, threads=8, timeout=None):
                    ASAN_OPTIONS="detect_leaks=0:detect_stack_use_after_return=0:abort_on_error=1",
                    UBSAN_OPTIONS="print_stacktrace=1:halt_on_error=1")
         t = time.perf_counter()
-        r = subprocess.run([exe, fin, fout], env=env, capture_output=True, text=True, timeout=timeout)
+        r = subprocess.run([exe, fin, fout, str(max_leaf), repr(traversal_cost)], env=env, capture_output=True, text=True, timeout=timeout)
         wall = time.perf_counter() - t
         if r.returncode != 0:
             raise RuntimeError(f"CPU execution of the device BVH build failed ({r.returncode}):\n{r.stderr[-4000:]}")

@@ -34,12 +34,12 @@ def _soup(tris):
     return s
 
 
-def _check(exe, scene):
-    scene.build()
+def _check(exe, scene, **build):
+    scene.build(**build)
     r = scene.raw()
     p = np.ctypeslib.as_array(r.positions, (r.num_vertices * 3,)).reshape(-1, 3).copy() if r.num_vertices else np.zeros((0, 3), np.float32)
     i = np.ctypeslib.as_array(r.indices, (r.num_tris * 3,)).reshape(-1, 3).copy() if r.num_tris else np.zeros((0, 3), np.int32)
-    nodes, order, stats, _ = hipcpu_run.run(exe, p, i, timeout=600)
+    nodes, order, stats, _ = hipcpu_run.run(exe, p, i, timeout=600, **build)
     st = gpu.BvhBuildStats.from_buffer_copy(stats)
     hs = scene.stats()
     assert nodes.tobytes() == scene.nodes().tobytes()
@@ -58,6 +58,15 @@ def test_random_soups_across_the_thresholds(exe):
     for n in (1, 2, 3, 9, 2047, 2048, 2049, 6000):
         c = g.uniform(-10, 10, (n, 1, 3))
         _check(exe, _soup(c + g.normal(0, 0.3, (n, 3, 3))))
+
+
+@pytest.mark.parametrize("max_leaf,cost", [(255, 1e9), (256, 1e9), (300, 50.0), (1000, 1e9), (1000, 200.0), (2100, 1e9)])
+def test_leaves_above_the_subtree_bound(exe, max_leaf, cost):
+    """Leaves larger than the subtrees that one block builds (256 triangles here): nodes that the host splits level by
+    level become leaves there."""
+    g = np.random.default_rng(13)
+    c = g.uniform(-10, 10, (4500, 1, 3))
+    _check(exe, _soup(c + g.normal(0, 0.3, (4500, 3, 3))), max_leaf=max_leaf, traversal_cost=cost)
 
 
 def test_degenerate_layouts(exe):

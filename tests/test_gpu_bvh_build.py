@@ -19,10 +19,10 @@ def _mesh(scene):
     return p, i
 
 
-def _compare(scene):
-    scene.build()
+def _compare(scene, **build):
+    scene.build(**build)
     p, i = _mesh(scene)
-    nodes, order, st = gpu.bvh_build(p, i)
+    nodes, order, st = gpu.bvh_build(p, i, **build)
     want = scene.nodes()
     hs = scene.stats()
     print(f"{len(i)} triangles: {len(want)} nodes, device build {st.build_ms:.1f} ms, host {hs.build_ms:.1f} ms")
@@ -46,6 +46,12 @@ def test_builtin_scenes(name):
 def test_sphere_soup_and_field():
     _compare(host.Scene.spheres(256, box=100.0, alpha_fraction=0.1, seed=1))
     _compare(host.Scene.field(64, seed=3, env_width=64))
+
+
+@pytest.mark.parametrize("spheres", [4, 64, 128])
+@pytest.mark.parametrize("max_leaf,cost", [(300, 50.0), (1000, 1e9), (2100, 1e9)])
+def test_leaves_above_the_subtree_bound(spheres, max_leaf, cost):
+    _compare(host.Scene.spheres(spheres, box=60.0, seed=2), max_leaf=max_leaf, traversal_cost=cost)
 
 
 @pytest.mark.skip(reason="a 1M-triangle device build with an earlier subtree kernel made a GPU memory fault whose cause was not "
