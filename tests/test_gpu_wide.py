@@ -139,3 +139,93 @@ def test_any_hit_launches_report_the_same_hits(n):
     want, _ = trace_on_gpu(r, rays, anyhit=True, counts=True)
     assert got.tobytes() == want.tobytes()
     r.close()
+
+
+def _lit(**kw):
+    """A _mesh scene with light from a sky of one colour and from its first triangles, and a camera that sees it."""
+    rng = np.random.default_rng(11)
+    n, twice, max_leaf = kw.get("n", 300), kw.get("twice", False), kw.get("max_leaf", 0)
+    p = (rng.uniform(-1, 1, (n, 1, 3)) + rng.normal(0, 0.15, (n, 3, 3))).reshape(-1, 3).astype(np.float32)
+    s = host.Scene()
+    dull, lamp = Material.default(), Material.default()
+    dull.base_color[:], dull.metallic, dull.double_sided = (0.7, 0.6, 0.5, 1.0), 0.0, 1
+    lamp.emission[:], lamp.double_sided = (8.0, 7.0, 6.0), 1
+    a, b = s.add_material(dull), s.add_material(lamp)
+    for _ in range(2 if twice else 1):
+        s.add_mesh(p, np.arange(len(p), dtype=np.int32), a)
+    q = (rng.uniform(-1.5, 1.5, (6, 1, 3)) + rng.normal(0, 0.3, (6, 3, 3))).reshape(-1, 3).astype(np.float32)
+    s.add_mesh(q, np.arange(len(q), dtype=np.int32), b)
+    s.set_env_color((0.3, 0.4, 0.5), 1.0)
+    s.set_camera((0.2, 0.3, 4.0), (0, 0, 0), (0, 1, 0), 45.0)
+    return s.build(max_leaf=max_leaf, traversal_cost=1e9 if max_leaf > 32 else 0.0)
+
+
+@pytest.mark.parametrize("kw", [dict(max_leaf=100), dict(twice=True), dict()], ids=["no-wide-nodes", "every-triangle-twice", "plain"])
+def test_every_path_renders_the_same_image(kw):
+    """One image through every kernel that traces paths: the per-pixel one, a sample per lane, bounces over few slots,
+    bounces that end one path per thread, the binary nodes' top staged in LDS, and serving among other jobs. Leaves of
+    100 triangles have no wide nodes: all of it walks the binary ones. Where every triangle is there twice, every hit is a
+    tie that the wide walk leaves to the binary one, in the queues' second pass too."""
+    from oracle import oracle_py
+
+    scene = _lit(**kw)
+    w, h, spp = 90, 61, 4
+    rs, cam = RenderSettings.make(w, h, max_depth=6, rr_depth=3, seed=3), scene.camera_view(w / h)
+    images = {}
+
+    def accum(r):
+        return gpu.copy_device_to_numpy(r.buffer_ptr(gpu.BUF_ACCUM), w * h * 16, np.float32).tobytes()
+
+    for name, engine, cfg in (("per-pixel", gpu.ENGINE_MEGAKERNEL, {}), ("direct", gpu.ENGINE_WAVEFRONT, {}),
+                              ("bounces", gpu.ENGINE_WAVEFRONT, dict(path_slots=1000, finish_percent=0)),
+                              ("finished", gpu.ENGINE_WAVEFRONT, dict(path_slots=3000, finish_percent=100)),
+                              ("samples", gpu.ENGINE_WAVEFRONT, dict(path_slots=5000, sample_split=4, refill_lanes=1, finish_percent=0)),
+                              ("top", gpu.ENGINE_WAVEFRONT, dict(path_slots=1000, lds_nodes=16, finish_percent=0))):
+        r = uploaded(scene, w, h, engine=engine)
+        if cfg:
+            r.set_wavefront_config(**cfg)
+        r.render(cam, rs, spp)
+        images[name] = accum(r)
+        if name == "per-pixel":
+            image = r.download_image()
+            ref = oracle_py.render(scene.desc(), cam, rs, spp)
+            assert np.mean(np.all(np.abs(image - ref) <= 1e-3 * np.abs(ref) + 1e-6, axis=2)) >= 0.999
+            assert image.mean() > 0.05
+        r.close()
+    for name in images:
+        assert images[name] == images["per-pixel"], name
+    srv = gpu.Server(path_slots=2000, express_slots=-1, min_items=1)
+    other = host.Scene.builtin("materials").build()
+    a, b = srv.add_scene(scene), srv.add_scene(other)
+    jobs = [srv.submit(a, w, h, spp, cam, max_depth=6, seed=3), srv.submit(b, 64, 40, 3, other.camera_view(1.6), max_depth=6, seed=9)]
+    srv.run_until_idle()
+    assert srv.result(jobs[0]).tobytes() == image.tobytes()
+    alone = gpu.Server(path_slots=2000, express_slots=-1, min_items=1)
+    j = alone.submit(alone.add_scene(other), 64, 40, 3, other.camera_view(1.6), max_depth=6, seed=9)
+    alone.run_until_idle()
+    assert alone.result(j).tobytes() == srv.result(jobs[1]).tobytes()
+    alone.close()
+    srv.close()
+
+
+@pytest.mark.parametrize("kw", [dict(max_leaf=100), dict(twice=True)], ids=["no-wide-nodes", "every-triangle-twice"])
+def test_real_time_samples_of_scenes_left_to_the_binary_nodes(kw):
+    """The one-sample G-buffer kernels: the compact sample's colour is the first sample of the render, and the denoised
+    frame traces the same one."""
+    scene = _lit(**kw)
+    w, h = 75, 50
+    rs, cam = RenderSettings.make(w, h, max_depth=5, rr_depth=3, seed=6), scene.camera_view(w / h)
+    r = uploaded(scene, w, h)
+    r.render(cam, rs, 1)
+    first = r.download_image()
+    r.close()
+    r = uploaded(scene, w, h)
+    g = gpu.CompactGBuffer(w, h)
+    r.sample_compact(cam, rs, g)
+    assert g.planes["color"].numpy(np.float32, (h, w, 3)).tobytes() == first.tobytes()
+    r.close()
+    r = uploaded(scene, w, h)
+    r.render_denoised(cam, cam, rs)
+    colour = gpu.copy_device_to_numpy(r.buffer_ptr(gpu.BUF_COLOR), w * h * 16, np.float32, (h, w, 4))
+    assert np.ascontiguousarray(colour[..., :3]).tobytes() == first.tobytes()
+    r.close()
