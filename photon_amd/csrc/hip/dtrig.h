@@ -3,9 +3,10 @@
 // The arguments are bounded (angles of warps within [-2 pi, 2 pi], unit directions), so the general library
 // functions' wide argument reduction and extended-precision branches are not needed: they are what held the
 // shading kernels' registers. Argument reduction by pi/2 in two parts with fused multiply-adds, then Taylor
-// polynomials on [-pi/4, pi/4]; the arctangent is reduced to |t| <= tan(pi/8) and evaluated with the polynomial
-// that interpolates it at 12 Chebyshev nodes (error 2e-19). Each fp64 value is within about 2 units in its last
-// place, so the fp32 results are the correctly rounded ones except with a probability of about 2^-27 per call.
+// polynomials on [-pi/4, pi/4]; the arctangent is reduced to |t| <= tan(pi/8) and evaluated with a polynomial
+// that interpolates it at 12 Chebyshev nodes (error below 1.5e-18, a thirtieth of a unit). Each fp64 value is within 2 units in its last place,
+// the arccosine's, which comes from an arctangent of a square root, within 3 (its error, and the others', measured
+// against numpy: tests/test_trig_cpu.py), so the fp32 results are the correctly rounded ones except with a probability of about 2^-27 per call.
 #pragma once
 
 #include <stdint.h>
@@ -75,9 +76,7 @@ PH_DEV void sincos_cr(float x, float* s, float* c) {
 }
 PH_DEV float atan2_cr(float y, float x) { return float(atan2_64(double(y), double(x))); }
 // x in [-1, 1].
-PH_DEV float acos_cr(float x) {
-    const double d = double(x);
-    return float(atan2_64(__builtin_sqrt((1.0 - d) * (1.0 + d)), d));
-}
+PH_DEV double acos64(double x) { return atan2_64(__builtin_sqrt((1.0 - x) * (1.0 + x)), x); }
+PH_DEV float acos_cr(float x) { return float(acos64(double(x))); }
 
 }  // namespace phd
