@@ -29,19 +29,18 @@ METRIC = "Msamples/s at 1080p 64spp; traversal Mrays/s; request p50/p99 latency"
 # 80 + 12 + 24 + 16 per alpha test (material, indices, uvs, 4 texels).
 RAY_IO, NODE_B, TRI_B, ALPHA_B = 28 + 16, 64, 48, 80 + 12 + 24 + 16
 # Algorithmic bytes of one SVGF frame per pixel with the 16-byte planes the denoiser reads: each pass
-# reads its distinct inputs once and writes its outputs once. temporal: 5 current planes + 4 history
-# planes in, illumination + moments out (11 x 16); variance: illumination, moments, normal, position in,
-# 1 out (5 x 16); five a-trous passes: filtered, normal, position in, 1 out (4 x 16 each); history:
-# filtered, illumination, moments, normal, position in, 4 out (9 x 16); remodulate: filtered, colour,
-# albedo, emission, position in, 1 out (6 x 16). Total 816 bytes.
-SVGF_BYTES_PER_PIXEL = 11 * 16 + 5 * 16 + 5 * 4 * 16 + 9 * 16 + 6 * 16
+# reads its distinct inputs once and writes its outputs once, with a settled history. temporal: 5 current
+# planes + 4 history planes in, illumination, moments, filter plane and packed material out (12 x 16 + 4);
+# variance: nothing; five a-trous passes: filtered, normal, packed material in, 1 out (3 x 16 + 4 each);
+# history: filtered, illumination, moments, normal, position in, 4 out (9 x 16); remodulate: filtered, colour,
+# albedo, emission, packed material in, 1 out (5 x 16 + 4). Total 684 bytes.
+SVGF_BYTES_PER_PIXEL = 12 * 16 + 4 + 5 * (3 * 16 + 4) + 9 * 16 + 5 * 16 + 4
 # The same count for the workload's compact G-buffer (12-byte colour, albedo and emission, 4-byte depth,
 # normal code and material; float4 internal planes; the previous frame's geometry kept as depth, normal
-# code and material). temporal: 48 current + 44 history in, 32 out (124); variance: illumination,
-# moments, geometry in, 1 out (60); a-trous: filtered + geometry in, 1 out (44 each); history: filtered,
-# illumination, moments, geometry in, 44 out (104); remodulate: material, filtered, albedo, emission,
-# colour in, 1 out (72). Total 580 bytes.
-SVGF_COMPACT_BYTES_PER_PIXEL = 124 + 60 + 5 * 44 + 104 + 72
+# code and material). temporal: 48 current + 44 history in, 48 out (140); variance: nothing; a-trous: filtered +
+# geometry in, 1 out (44 each); history: filtered, illumination, moments, geometry in, 44 out (104);
+# remodulate: material, filtered, albedo, emission, colour in, 1 out (72). Total 536 bytes.
+SVGF_COMPACT_BYTES_PER_PIXEL = 140 + 5 * 44 + 104 + 72
 
 
 # Algorithmic bytes of a path vertex beyond its rays (per sample: the scope table's B_sample): a shading

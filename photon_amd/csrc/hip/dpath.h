@@ -38,9 +38,6 @@ struct RayTally {
     unsigned ext, shadow;
 };
 
-// The path from its next extension ray (ro, rd) on, with the generator in the state it has at that
-// point: the remaining vertices exactly as a path that started here would run them. trace_path is the
-// whole path; the wavefront engine resumes its last paths in flight with this.
 // The stack of a kernel that traces whole paths: 16 KB of LDS per 128 lanes for either walk.
 template <int Block, bool Wide>
 using PathStack = StackShape<Block, Wide ? 20 : 32, Wide>;
@@ -57,6 +54,9 @@ PH_DEV bool path_query(const DScene& s, f3 o, f3 d, float tmax, HitRec& hit, Lan
     return traverse<AnyHit, Count>(s, o, d, tmax, hit, stack, cnt);
 }
 
+// The path from its next extension ray (ro, rd) on, with the generator in the state it has at that
+// point: the remaining vertices exactly as a path that started here would run them. trace_path is the
+// whole path; the wavefront engine resumes its last paths in flight with this.
 template <class Stack, bool Count>
 PH_DEV f3 trace_path_from(const DScene& s, f3 ro, f3 rd, Pcg& rng, const PathOpts& opt, PathState ps, PrimaryOut* primary, Stack& stack,
                           TraceCount* cnt, RayTally* tally) {

@@ -4,9 +4,10 @@
 // functions' wide argument reduction and extended-precision branches are not needed: they are what held the
 // shading kernels' registers. Argument reduction by pi/2 in two parts with fused multiply-adds, then Taylor
 // polynomials on [-pi/4, pi/4]; the arctangent is reduced to |t| <= tan(pi/8) and evaluated with a polynomial
-// that interpolates it at 12 Chebyshev nodes (error below 1.5e-18, a thirtieth of a unit). Each fp64 value is within 2 units in its last place,
-// the arccosine's, which comes from an arctangent of a square root, within 3 (its error, and the others', measured
-// against numpy: tests/test_trig_cpu.py), so the fp32 results are the correctly rounded ones except with a probability of about 2^-27 per call.
+// that interpolates it at 12 Chebyshev nodes (error below 1.5e-18, a thirtieth of a unit). Each fp64 value is within
+// 2 units in its last place, the arccosine's, which comes from an arctangent of a square root, within 3 (measured
+// against numpy: tests/test_trig_cpu.py), so the fp32 results are the correctly rounded ones except with a
+// probability of about 2^-27 per call.
 #pragma once
 
 #include <stdint.h>

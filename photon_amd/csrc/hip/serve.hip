@@ -14,7 +14,7 @@
 // set by its own depth rather than by iterations over millions of other paths.
 //
 // A job with fewer than `min_items` pixels runs each pixel's samples as S sub-streams (S divides spp)
-// in separate partial images, which the result adds in sub-stream order: its paths can then fill more
+// in separate partial sums, which the result adds in sub-stream order: its paths can then fill more
 // slots than it has pixels. Within a sub-stream the samples are taken in order, pass after pass. An
 // image therefore depends only on the job and the server's configuration, never on what else shared
 // the wavefronts; with S = 1 it is bit-identical to the renderer's.

@@ -24,7 +24,7 @@ struct WavefrontJob {
     float4* nd;
     const int* mat_class;  // per-material class table in device memory (nullptr: computed per render)
     // Serving: the samples of each pixel run as `split` sub-streams of spp / split samples, each added
-    // to its own partial image (accum holds split planes of width x height); 1 for the renderer.
+    // to its own partial sum (accum[pixel * split + sub-stream]); 1 for the renderer.
     int split = 1;
 };
 

@@ -104,7 +104,7 @@ struct State {
     int* pixel;
     int* sample;
     int* sample_end;  // end of the slot's pass (serving)
-    int* part;        // the slot's sub-stream (serving: accumulates into partial image `part`)
+    int* part;        // the slot's sub-stream (serving: sums into partial sum `part` of its pixel)
     uint8_t* stage;
     uint64_t* rng;
     float4* ro;  // origin, prev_pdf
@@ -1375,7 +1375,8 @@ ph_wavefront_config WavefrontEngine::config() const { return impl_->cfg; }
 // whole samples, every sample of a chunk its own work item. The partial sums are single samples, added in sample
 // order, so the image is the in-order one bit for bit, and a chunk lasts as long as its longest paths, not as long as
 // the pixel with the longest run of them. 853x479, 8 samples of the materials scene: 3.5 ms, 11.8 with one item a
-// pixel; the 1M-triangle field's geometry at 1080p x 64 about 61 ms, 110 before. kChunkItems bounds the partial sums
+// pixel; 1080p x 64 over the 65,538-triangle field 41 ms, 107 before, over the 1M-triangle one 81 and 197. A million
+// samples with paths of up to 64 vertices and no roulette take 4.1 ms in either form (4.7 with one item a pixel). kChunkItems bounds the partial sums
 // (1 GB) and kChunkSlots the paths' state (1.6 GB; at 4M slots the field takes 68 ms). Two bounces a graph: a bounce
 // that finds nothing costs 0.1 ms, a look at the queue 0.03. Chunks of at most kDirectItems samples run a sample per
 // lane: 64x64x4 Cornell box 0.32 ms (0.65 in bounces), 320x240x12 glass 1.56 (1.81), 640x360x4 materials 1.49 (2.1),
