@@ -68,10 +68,6 @@ struct DevBuf {
         PH_CHECK(e);
         count = n;
     }
-    // At least n elements: grows, never shrinks.
-    void reserve(size_t n) {
-        if (n > count) allocate(n);
-    }
     void upload(const void* src, size_t n, hipStream_t st) {
         allocate(n);
         if (n) PH_CHECK(hipMemcpyAsync(ptr, src, n * sizeof(T), hipMemcpyHostToDevice, st));

@@ -17,12 +17,14 @@ struct PathBuffers {
     DevBuf<uint8_t> stage;
     DevBuf<uint64_t> rng;
     DevBuf<float4> ro, rd, beta, L, hit, so, sd, sc;
+    DevBuf<float4> part_sums;  // partial sums of a single render in sub-streams
     int capacity = 0;  // slots that every array has room for
 
     // Renders of changing sizes keep the largest one's arrays, up to this many slots (1.6 GB): 1920x1080 Cornell with 1 and
     // 4 samples in turn takes 3.9 ms a pair, 16.4 with arrays of the exact size. What a configuration asked
     // for beyond that is given back by the next smaller call.
     static constexpr int kKeptSlots = 1 << 23;
+    static constexpr size_t kKeptSums = size_t(1) << 26;  // the same for partial sums (1 GB)
 
     // Whether make_room(n) would allocate (what points into the arrays is to be dropped before).
     bool moves(int n) const { return n > capacity || (n < capacity && capacity > kKeptSlots); }
@@ -41,8 +43,14 @@ struct PathBuffers {
         capacity = n;
     }
 
+    // Room for at least n partial sums.
+    void make_sums(size_t n) {
+        if (n > part_sums.count || part_sums.count > kKeptSums) part_sums.allocate(n);
+    }
+
     void release() {
         capacity = 0;
+        part_sums.release();
         for (DevBuf<int>* b : {&job, &pixel, &sample, &sample_end, &part, &q_ext, &q_shadow, &q_term, &q_miss, &partial, &first_pos}) b->release();
         for (auto& q : q_cls) q.release();
         stage.release();

@@ -1076,7 +1076,6 @@ struct WavefrontEngine::Impl : PathBuffers {
     DevBuf<long long> chunk_first;
     DevBuf<unsigned long long> items;  // next work item, items queued
     DevBuf<int4> chunk_pass;
-    DevBuf<float4> part_sums;  // partial sums of a single render in sub-streams
     DevBuf<unsigned long long> direct_rays;  // direct_kernel's tallies
     DevBuf<JobParams> jobs;
     DevBuf<TraceTotals> totals;             // [0] extension rays, [1] shadow rays
@@ -1158,7 +1157,6 @@ struct WavefrontEngine::Impl : PathBuffers {
     void give_back() {
         drop_graph();
         release();
-        part_sums.release();
     }
 
     State state() {
@@ -1422,7 +1420,7 @@ void WavefrontEngine::render_direct(hipStream_t st, const WavefrontJob& job, ph_
     WavefrontJob sub = job;
     sub.split = job.spp;
     if (sub.split > 1) {
-        m.part_sums.reserve(size_t(items));
+        m.make_sums(size_t(items));
         sub.accum = m.part_sums.ptr;
     }
     m.direct_rays.allocate(2 * kDirectTallies);
@@ -1456,7 +1454,7 @@ void WavefrontEngine::render_chunk(hipStream_t st, const WavefrontJob& job, int 
     WavefrontJob sub = job;
     sub.split = split;
     if (split > 1) {
-        m.part_sums.reserve(size_t(items));
+        m.make_sums(size_t(items));
         sub.accum = m.part_sums.ptr;
     }
     const JobParams jp = m.params_of(sub, job.mat_class ? job.mat_class : m.mat_class.ptr);

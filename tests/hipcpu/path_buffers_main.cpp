@@ -72,6 +72,15 @@ static void sizes_in_turn() {
     b.capacity = PathBuffers::kKeptSlots + 1;  // as if so many had been asked for
     b.make_room(4000);
     EXPECT(b.capacity == 4000 && holds(b, 4000) && b.ro.count == 4000);
+    b.make_sums(1000);
+    first = hipcpu::mallocs_made;
+    for (size_t n : {400, 1000, 1}) b.make_sums(n);
+    EXPECT(hipcpu::mallocs_made == first && b.part_sums.count == 1000);
+    b.make_sums(PathBuffers::kKeptSums + 1);
+    b.make_sums(500);
+    EXPECT(b.part_sums.count == 500);
+    b.release();
+    EXPECT(b.capacity == 0 && !b.part_sums.ptr && !b.ro.ptr && !b.q_cls[0].ptr);
 }
 
 // A render in chunks where at most `room` slots and items fit: every sample runs once, in order, in chunks that fit.
