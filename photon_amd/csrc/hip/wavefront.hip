@@ -1080,6 +1080,7 @@ struct WavefrontEngine::Impl : PathBuffers {
     DevBuf<JobParams> jobs;
     DevBuf<TraceTotals> totals;             // [0] extension rays, [1] shadow rays
     DevBuf<unsigned long long> ray_totals;  // rays traced: [0] extension, [1] shadow; finish_kernel: [2] extension, [3] shadow, [4] paths
+    void* host_block = nullptr;  // pinned, what the pointers below point into
     int* host_counters = nullptr;
     int* host_done = nullptr;
     int* host_sizes = nullptr;
@@ -1112,12 +1113,16 @@ struct WavefrontEngine::Impl : PathBuffers {
     int64_t total_work = 0;  // end of the item layout
 
     Impl() {
-        PH_CHECK(hipHostMalloc(reinterpret_cast<void**>(&host_counters), C_COUNT * sizeof(int), hipHostMallocDefault));
-        PH_CHECK(hipHostMalloc(reinterpret_cast<void**>(&host_done), kMaxJobs * sizeof(int), hipHostMallocDefault));
-        PH_CHECK(hipHostMalloc(reinterpret_cast<void**>(&host_sizes), 2 * sizeof(int), hipHostMallocDefault));
-        PH_CHECK(hipHostMalloc(reinterpret_cast<void**>(&host_items), 2 * sizeof(unsigned long long), hipHostMallocDefault));
-        PH_CHECK(hipHostMalloc(reinterpret_cast<void**>(&host_stage), 2 * sizeof(unsigned long long), hipHostMallocDefault));
-        PH_CHECK(hipHostMalloc(reinterpret_cast<void**>(&host_direct), 2 * kDirectTallies * sizeof(unsigned long long), hipHostMallocDefault));
+        // One pinned block: with six, a server (two engines) took 0.55 ms to create and 1.63 to close, now 0.23 and 0.23; a
+        // renderer 107 and 110 us, now 47 and 67.
+        constexpr size_t kWords = 4 + 2 * kDirectTallies, kInts = C_COUNT + kMaxJobs + 2;
+        PH_CHECK(hipHostMalloc(&host_block, kWords * sizeof(unsigned long long) + kInts * sizeof(int), hipHostMallocDefault));
+        host_items = static_cast<unsigned long long*>(host_block);
+        host_stage = host_items + 2;
+        host_direct = host_stage + 2;
+        host_counters = reinterpret_cast<int*>(host_direct + 2 * kDirectTallies);
+        host_done = host_counters + C_COUNT;
+        host_sizes = host_done + kMaxJobs;
         std::memset(host_items, 0, 2 * sizeof(unsigned long long));
         counters.allocate(C_COUNT);
         jobs.allocate(kMaxJobs);
@@ -1135,12 +1140,7 @@ struct WavefrontEngine::Impl : PathBuffers {
     ~Impl() {
         drop_graph();
         for (hipEvent_t e : events) (void)hipEventDestroy(e);
-        if (host_counters) (void)hipHostFree(host_counters);
-        if (host_done) (void)hipHostFree(host_done);
-        if (host_sizes) (void)hipHostFree(host_sizes);
-        if (host_items) (void)hipHostFree(host_items);
-        if (host_stage) (void)hipHostFree(host_stage);
-        if (host_direct) (void)hipHostFree(host_direct);
+        if (host_block) (void)hipHostFree(host_block);
     }
 
     void drop_graph() {
