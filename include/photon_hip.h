@@ -52,8 +52,9 @@ typedef struct ph_gpu_info {
 typedef struct ph_wavefront_config {
     int32_t block;         /* threads per block of the traversal kernels: 64, 128, 256 */
     int32_t stack_depth;   /* LDS stack entries per lane: 8, 16, 24, 32, 64 (rest spills to scratch). Of the walk over the
-                              binary nodes: the four-wide nodes, which a render walks where the scene has them and
-                              lds_nodes is 0, take 12 whatever is set */
+                              binary nodes: the four-wide nodes, which a render walks where the scene has them,
+                              lds_nodes is 0 and, unless path_slots is 0 and sample_split 1, its hierarchy has more than
+                              512 nodes, take 12 whatever is set */
     int32_t path_slots;    /* paths in flight (0: one per pixel, at most 4M; with sample_split 1 as well, the render's size
                               decides: chunks of whole samples, each sample a work item, over up to 8M paths (1.6 GB, and
                               1 GB of partial sums; less where the device has less), with the same image. Up to 2^20

@@ -1089,8 +1089,9 @@ struct WavefrontEngine::Impl : PathBuffers {
     unsigned long long* host_direct = nullptr;  // direct_kernel's tallies
     std::vector<hipEvent_t> events;
     hipGraphExec_t graph_exec = nullptr;
-    std::tuple<int, int, int, int, int, bool, bool> graph_key{};
-    bool wide = false;  // rays walk the wide nodes, which every scene in work has
+    std::tuple<int, int, int, int, int, bool, bool, bool> graph_key{};
+    bool wide = false;         // every scene in work has wide nodes
+    bool queues_wide = false;  // the queues' rays walk them (kFewNodes)
     std::map<std::tuple<const void*, int, int, int, int>, ph_wavefront_config> tuned;
     // Serving bookkeeping (host side).
     bool serving = false;
@@ -1222,7 +1223,7 @@ struct WavefrontEngine::Impl : PathBuffers {
         // find nothing cost it more (1280x720x4 Cornell job 2.80 ms, 2.84 with four; the mixed stream 26.2 either way).
         // Never more lanes than slots: a queue holds no more.
         const auto blocks_for = [&](int most, int block) { return std::max(1, std::min(most, (slots + block - 1) / block)); };
-        const bool over_wide = wide && !count && (Multi || cfg.lds_nodes == 0);
+        const bool over_wide = queues_wide && !count && (Multi || cfg.lds_nodes == 0);
         const int tgrid = blocks_for(cus * std::max(1, cfg.blocks_per_cu) * (over_wide && !Multi ? 4 : 1), cfg.block);
         // Shading: 4 blocks of 256 threads per CU, all of them resident: the shading kernels need 140 VGPRs since the
         // bounded trigonometry (dtrig.h; 232 before, 2 waves per SIMD), and 128 spill at most 8. 1080p, 64 samples, 1M
@@ -1234,7 +1235,7 @@ struct WavefrontEngine::Impl : PathBuffers {
         hipLaunchKernelGGL(bookkeep_kernel, dim3(1), dim3(64), 0, st, cnt, ray_totals.ptr);
         if (ev) PH_CHECK(hipEventRecord(ev[0], st));
         const int refill = std::clamp(cfg.refill_lanes, 1, 64);
-        fns.extend(st, tgrid, w, s, cnt, cfg.sort_materials ? 1 : 0, refill, cfg.lds_nodes, totals.ptr, count, wide);
+        fns.extend(st, tgrid, w, s, cnt, cfg.sort_materials ? 1 : 0, refill, cfg.lds_nodes, totals.ptr, count, queues_wide);
         if (ev) PH_CHECK(hipEventRecord(ev[1], st));
         compact<K_HIT, Multi>(st, s);
         hipLaunchKernelGGL(miss_kernel<Multi>, dim3(sgrid), dim3(256), 0, st, w, s, cnt);
@@ -1245,7 +1246,7 @@ struct WavefrontEngine::Impl : PathBuffers {
         hipLaunchKernelGGL((shade_kernel<7, Multi>), dim3(sgrid), dim3(256), 0, st, w, s, cnt, 3, bins);
         compact<K_DONE, Multi>(st, s);
         if (ev) PH_CHECK(hipEventRecord(ev[2], st));
-        fns.shadow(st, tgrid, w, s, cnt, 0, refill, cfg.lds_nodes, totals.ptr + 1, count, wide);
+        fns.shadow(st, tgrid, w, s, cnt, 0, refill, cfg.lds_nodes, totals.ptr + 1, count, queues_wide);
         if (ev) PH_CHECK(hipEventRecord(ev[3], st));
         hipLaunchKernelGGL(regen_kernel<Multi>, dim3(sgrid), dim3(256), 0, st, w, s, cnt);
         hipLaunchKernelGGL(advance_items_kernel, dim3(1), dim3(64), 0, st, items.ptr, cnt);
@@ -1272,7 +1273,7 @@ struct WavefrontEngine::Impl : PathBuffers {
         const ShapeFns fns = shapes(multi);
         const bool graph = cfg.use_graph != 0 && !counting;
         if (graph) {
-            auto key = std::make_tuple(cfg.block, cfg.stack_depth, cfg.blocks_per_cu, G, slots, multi, wide);
+            auto key = std::make_tuple(cfg.block, cfg.stack_depth, cfg.blocks_per_cu, G, slots, multi, wide, queues_wide);
             if (!graph_exec || key != graph_key) {
                 drop_graph();
                 hipGraph_t g = nullptr;
@@ -1369,6 +1370,19 @@ void WavefrontEngine::set_config(const ph_wavefront_config& c) {
 
 ph_wavefront_config WavefrontEngine::config() const { return impl_->cfg; }
 
+// The queues' rays of serving jobs, and of renders that are told their slots or sub-streams, walk the binary nodes where all
+// scenes in work have few (or one has no others): each bounce waits for its longest rays, and where a walk is short the wide
+// one's longer steps make those longer. Over wide and over binary nodes, jobs of 64x64x1 / 1280x720x4 and a render of
+// 1280x720x8 in single samples over 3.7M slots, ms: 17 nodes (Cornell box) 1.12 / 3.59 / 3.19 and 1.02 / 3.33 / 3.11; 247
+// nodes 0.83 / 2.25 / 2.51 and 0.81 / 2.23 / 2.46; 495 nodes 0.86 / 2.35 / 2.58 and 0.84 / 2.32 / 2.55; 996 nodes 0.91 /
+// 2.52 / 2.67 and 0.89 / 2.55 / 2.71; 3,968 nodes 1.00 / 2.91 / 2.96 and 0.99 / 2.99 / 3.10. At the default launch wide
+// nodes are faster or level at every size (Cornell 1280x720x8 2.17, binary 2.26; 1920x1080x1 1.22, 1.21).
+constexpr int kFewNodes = 512;
+
+bool queues_walk_wide(const ph_wavefront_config& c, const WavefrontJob& job) {
+    return job.scene.wide && (default_launch(c) || job.scene.num_nodes > kFewNodes);
+}
+
 // Launch rule of the default configuration (no path slots or sub-streams asked for): the render runs in chunks of
 // whole samples, every sample of a chunk its own work item. The partial sums are single samples, added in sample
 // order, so the image is the in-order one bit for bit, and a chunk lasts as long as its longest paths, not as long as
@@ -1447,6 +1461,7 @@ void WavefrontEngine::render_chunk(hipStream_t st, const WavefrontJob& job, int 
     const int slots = int(std::min(most, items));
     m.ensure_slots(slots);
     m.wide = job.scene.wide != nullptr;
+    m.queues_wide = queues_walk_wide(m.cfg, job);
     if (!job.mat_class) {
         std::vector<int> cls = material_classes(job.scene, st);
         m.mat_class.upload(cls.data(), cls.size(), st);
@@ -1531,7 +1546,7 @@ ph_wavefront_config WavefrontEngine::autotune(hipStream_t st, const WavefrontJob
     // One that would run the same launches is not timed: its reading could only differ by that spread, and a field that
     // this render does not look at would be kept for renders that do.
     auto launch_of = [&](const ph_wavefront_config& c) {
-        return effective_launch(c, int64_t(job.width) * job.height, job.spp, job.scene.wide != nullptr);
+        return effective_launch(c, int64_t(job.width) * job.height, job.spp, queues_walk_wide(c, job));
     };
     auto consider = [&](const ph_wavefront_config& c) {
         const ph_wavefront_config a = launch_of(c), b = launch_of(best);
@@ -1685,13 +1700,6 @@ void WavefrontEngine::serve_share(int quantum) {
     impl_->chunks_dirty = true;
 }
 
-// Serving walks the binary nodes if a scene in work has no others, and if all have few: each bounce waits for its longest
-// rays, and where a walk is short the wide one's longer steps make those longer. Jobs of 64x64x1 / 1280x720x4 over wide and
-// over binary nodes: 17 nodes (Cornell box) 1.12 / 3.59 ms and 1.02 / 3.33; 247 nodes 0.83 / 2.25 and 0.81 / 2.23; 996 nodes
-// 0.91 / 2.52 and 0.89 / 2.55; 3,968 nodes 1.00 / 2.91 and 0.99 / 2.99. (Renders at the default launch are faster over wide
-// nodes at every size.)
-constexpr int kFewNodes = 512;
-
 void WavefrontEngine::serve_run(hipStream_t st, int iterations) {
     Impl& m = *impl_;
     if (!m.serving) throw std::runtime_error("serve_begin was not called");
@@ -1767,7 +1775,8 @@ void WavefrontEngine::serve_run(hipStream_t st, int iterations) {
             least = std::min(least, m.entry_nodes[size_t(e)]);
             most = std::max(most, m.entry_nodes[size_t(e)]);
         }
-    m.wide = least > 0 && most > kFewNodes;
+    m.wide = least > 0;
+    m.queues_wide = m.wide && most > kFewNodes;
     m.run_batch(st, std::max(1, iterations), true, false);
     PH_CHECK(hipMemcpyAsync(m.host_done, m.job_done.ptr, kMaxJobs * sizeof(int), hipMemcpyDeviceToHost, st));
     PH_CHECK(hipStreamSynchronize(st));

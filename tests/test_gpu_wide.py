@@ -128,6 +128,25 @@ def test_wavefront_image_over_either_walk(w, h, spp, split):
     r.close()
 
 
+@pytest.mark.parametrize("n", [480, 900])
+def test_default_and_configured_launches_alternate(n):
+    """Hierarchies on either side of 512 nodes, the line up to which the queues of configured slots walk the binary nodes
+    and the default launch's the wide ones: one renderer, in turns, so that each has to find its own launches again."""
+    scene = _lit(n=n)
+    assert (scene.desc().num_nodes > 512) == (n == 900)
+    w, h, spp = 520, 512, 5  # more than 2^20 samples: the default launch runs in bounces
+    cam, rs = scene.camera_view(w / h), RenderSettings.make(w, h, max_depth=6, rr_depth=3, seed=4)
+    r = uploaded(scene, w, h, engine=gpu.ENGINE_WAVEFRONT)
+    default, images = r.wavefront_config(), []
+    for cfg in ({}, dict(path_slots=w * h * spp, sample_split=spp)) * 3:
+        r.set_wavefront_config(**(cfg or {f: getattr(default, f) for f, _ in default._fields_}))
+        r.reset()
+        r.render(cam, rs, spp)
+        images.append(gpu.copy_device_to_numpy(r.buffer_ptr(gpu.BUF_ACCUM), w * h * 16, np.float32).tobytes())
+    assert len(set(images)) == 1
+    r.close()
+
+
 @pytest.mark.parametrize("n", [1, 129, 786431, 786432, 1000003, 1966079, 1966080, 2500007])
 def test_any_hit_launches_report_the_same_hits(n):
     """Few any-hit rays run in blocks with deep stacks, more (from 786,432 on) in blocks with short ones, many (from 1,966,080
@@ -160,12 +179,14 @@ def _lit(**kw):
     return s.build(max_leaf=max_leaf, traversal_cost=1e9 if max_leaf > 32 else 0.0)
 
 
-@pytest.mark.parametrize("kw", [dict(max_leaf=100), dict(twice=True), dict()], ids=["no-wide-nodes", "every-triangle-twice", "plain"])
+@pytest.mark.parametrize("kw", [dict(max_leaf=100), dict(twice=True), dict(), dict(twice=True, n=900), dict(n=900)],
+                         ids=["no-wide-nodes", "every-triangle-twice", "plain", "every-triangle-twice-900", "plain-900"])
 def test_every_path_renders_the_same_image(kw):
     """One image through every kernel that traces paths: the per-pixel one, a sample per lane, bounces over few slots,
     bounces that end one path per thread, the binary nodes' top staged in LDS, and serving among other jobs. Leaves of
     100 triangles have no wide nodes: all of it walks the binary ones. Where every triangle is there twice, every hit is a
-    tie that the wide walk leaves to the binary one, in the queues' second pass too."""
+    tie that the wide walk leaves to the binary one, in the queues' second pass too. Of 900 triangles a hierarchy has more
+    than the 512 nodes up to which the queues of serving and of configured slots walk the binary ones."""
     from oracle import oracle_py
 
     scene = _lit(**kw)
